@@ -75,6 +75,6 @@ def build(name):
 
 
 if __name__ == "__main__":
-    names = sys.argv[1:] or [*PROGRAMS, *(REF_PROGRAMS if os.path.isdir(REFERENCE) else [])]
+    names = sys.argv[1:] or [*PROGRAMS, *(REF_PROGRAMS if os.path.isdir(os.path.join(REFERENCE, "apps")) else [])]
     for n in names:
         print(build(n), flush=True)
