@@ -113,6 +113,12 @@ int op2h_streaming(size_t stream_bytes);
 /* Pending launches taken over by a later stub since the library loaded. */
 unsigned long long op2h_fused_count(void);
 
+/* Called by op2h_graph_begin before the capture starts: a kernel file
+ * allocates and packs there what its launches inside a capture need (nothing
+ * may be allocated or uploaded once it has started). */
+typedef void (*op2h_capture_hook)(void);
+void op2h_register_capture_hook(op2h_capture_hook hook);
+
 /* A counter advanced whenever the runtime drops its plans (op_exit,
  * op_renumber): data a stub derives from a plan is valid while it holds. */
 unsigned op2h_plan_epoch(void);
@@ -139,6 +145,15 @@ void *op2h_gbl_slot(op2h_loop_ctx *ctx, int argi, int info_argi);
  * NULLs, and the stub finishes the reduction into op2h_gbl_slot itself. */
 int op2h_gbl_partials(op2h_loop_ctx *ctx, int argi, int info_argi, int nparts,
                       double **vals, int **locs);
+/* The same for an OP_INC arg whose partials are unevaluated pairs hi + lo
+ * (Sum2 of op2h_reduce.h): the result is their sum, rounded once, whatever the
+ * partials' number and order. */
+int op2h_gbl_partials2(op2h_loop_ctx *ctx, int argi, int nparts, double **hi,
+                       double **lo);
+/* A pending launch that writes only the first `nparts` of the partials at
+ * `vals` (a fused launch of another shape) says so when it is launched,
+ * before the graph's capture ends. */
+void op2h_gbl_partials_used(const double *vals, int nparts);
 
 /* Device scratch for per-workgroup partials and the zero-initialised
  * completion counter of the single-pass (last-workgroup-reduces) reduction.
@@ -357,8 +372,8 @@ int op2h_stream_probe(size_t bytes, int variant, int reps, double *gbs,
  * loop's own reductions over the cells (identity-started: rms sum 0, maxerr
  * -infinity) go to the caller's device struct `result`, on `stream` (NULL:
  * the default stream); the caller combines them with its own values.  It
- * allocates nothing: its per-workgroup partials (at most 2048, 20 bytes each)
- * live in a 40 KiB device array of the library, one per device, shared by all
+ * allocates nothing: its per-workgroup partials (at most 2048, 28 bytes each)
+ * live in a 56 KiB device array of the library, one per device, shared by all
  * calls on that device — calls that overlap on one device race.  No memset
  * and no host synchronisation, so the call can be captured into a graph.
  * block: 64..1024, a multiple of 64; ncell: any non-negative int.

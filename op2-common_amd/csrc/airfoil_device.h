@@ -8,6 +8,9 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
+
+#include "op2h_reduce.h"
 
 // ---------------------------------------------------------------------------
 // application constants (op_decl_const, airfoil.cpp:204-210)
@@ -187,6 +190,30 @@ __device__ __forceinline__ void update(const double *qold, double *q,
   }
 }
 
+// What res_calc computes of one cell alone, whatever the edge: ri = 1 / q[0]
+// and the pressure p, with its operations in its order.
+__device__ __forceinline__ void cell_terms(const double *q, double *ri, double *p) {
+  *ri = 1.0 / q[0];
+  *p = gm1_d * (q[3] - 0.5 * *ri * (q[1] * q[1] + q[2] * q[2]));
+}
+
+// Adds an edge's increment to one of its cells: +f of res_flux to ecell[0],
+// -f to ecell[1] (second), the same bits, with both cells' terms and the sum
+// of their adt given.  The sign goes into the factors that every term of f
+// has (0.5 and mu): negating both terms of a sum negates it exactly.
+template <class T>
+__device__ __forceinline__ void add_flux(T dx, T dy, const T *q1, T ri1, T p1, const T *q2, T ri2,
+                                         T p2, T adt, bool second, T eps, T *acc) {
+  const T half = second ? (T)-0.5 : (T)0.5;
+  const T vol1 = ri1 * (q1[1] * dy - q1[2] * dx);
+  const T vol2 = ri2 * (q2[1] * dy - q2[2] * dx);
+  const T mu = half * adt * eps;
+  acc[0] += half * (vol1 * q1[0] + vol2 * q2[0]) + mu * (q1[0] - q2[0]);
+  acc[1] += half * (vol1 * q1[1] + p1 * dy + vol2 * q2[1] + p2 * dy) + mu * (q1[1] - q2[1]);
+  acc[2] += half * (vol1 * q1[2] - p1 * dx + vol2 * q2[2] - p2 * dx) + mu * (q1[2] - q2[2]);
+  acc[3] += half * (vol1 * (q1[3] + p1) + vol2 * (q2[3] + p2)) + mu * (q1[3] - q2[3]);
+}
+
 }  // namespace op2_k
 
 // FP32 user kernels of the mixed-precision mode: the reference's
@@ -271,6 +298,11 @@ __device__ __forceinline__ void bres_calc(const float *x1, const float *x2,
     f = 0.5f * (vol1 * (q1[3] + p1) + vol2 * (qinf_f[3] + p2)) + mu * (q1[3] - qinf_f[3]);
     res1[3] += f;
   }
+}
+
+__device__ __forceinline__ void cell_terms(const float *q, float *ri, float *p) {
+  *ri = 1.0f / q[0];
+  *p = gm1_f * (q[3] - 0.5f * *ri * (q[1] * q[1] + q[2] * q[2]));
 }
 
 // The increment f of res_calc (SP), like op2_k::res_flux.
@@ -376,6 +408,54 @@ __device__ __forceinline__ int4 ld_int4_nt(const int *__restrict p, int n) {
   return make_int4(t.x, t.y, t.z, t.w);
 }
 
+// Rows in the arithmetic of the caller: FP64 rows as they are or rounded to
+// FP32 (mixed mode's x and q), FP32 rows (its adt and res)
+template <bool SOA>
+__device__ __forceinline__ void ld2r(const double *__restrict p, int n, int s, double *v) {
+  ld2<SOA>(p, n, s, v);
+}
+template <bool SOA>
+__device__ __forceinline__ void ld2r(const double *__restrict p, int n, int s, float *v) {
+  double t[2];
+  ld2<SOA>(p, n, s, t);
+  v[0] = (float)t[0];
+  v[1] = (float)t[1];
+}
+template <bool SOA>
+__device__ __forceinline__ void ld4r(const double *__restrict p, int n, int s, double *v) {
+  ld4<SOA>(p, n, s, v);
+}
+template <bool SOA>
+__device__ __forceinline__ void ld4r(const double *__restrict p, int n, int s, float *v) {
+  double t[4];
+  ld4<SOA>(p, n, s, t);
+  for (int d = 0; d < 4; ++d) v[d] = (float)t[d];
+}
+template <bool SOA>
+__device__ __forceinline__ void ld4r(const float *__restrict p, int n, int s, float *v) {
+  if (SOA) {
+    for (int d = 0; d < 4; ++d) v[d] = p[(size_t)d * s + n];
+  } else {
+    float4 a = *reinterpret_cast<const float4 *>(p + 4 * (size_t)n);
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = a.z;
+    v[3] = a.w;
+  }
+}
+template <bool SOA>
+__device__ __forceinline__ void st4r(double *__restrict p, int n, int s, const double *v) {
+  st4<SOA>(p, n, s, v);
+}
+template <bool SOA>
+__device__ __forceinline__ void st4r(float *__restrict p, int n, int s, const float *v) {
+  if (SOA) {
+    for (int d = 0; d < 4; ++d) p[(size_t)d * s + n] = v[d];
+  } else {
+    *reinterpret_cast<float4 *>(p + 4 * (size_t)n) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+}
+
 template <bool SOA>
 __device__ __forceinline__ void add4(double *__restrict p, int n, int s,
                                      const double *v) {
@@ -476,39 +556,58 @@ __device__ __forceinline__ void owner_apply(T *acc, const T *lf, int ent) {
   }
 }
 
+// The flux of one edge in the arithmetic of R (float: the mixed mode's).
+__device__ __forceinline__ void edge_flux(const double *x1, const double *x2, const double *q1,
+                                          const double *q2, double a1, double a2, double *f) {
+  op2_k::res_flux(x1, x2, q1, q2, a1, a2, f);
+}
+__device__ __forceinline__ void edge_flux(const float *x1, const float *x2, const float *q1,
+                                          const float *q2, float a1, float a2, float *f) {
+  op2_kf::res_flux(x1, x2, q1, q2, a1, a2, f);
+}
+
+// Phase 1 of an owner-compute block: one flux per edge touching the block
+// (edges on the block boundary are evaluated by both neighbouring blocks),
+// from global memory, into LDS lf[max_e][4].
+template <class R, bool SOA>
+__device__ __forceinline__ void owner_fluxes(int b, const double *__restrict x,
+                                             const double *__restrict q,
+                                             const R *__restrict adt, const OwnerArgs &P,
+                                             int sx, int sq, R *lf) {
+  const int e0 = P.elem_offs[b], ne = P.elem_offs[b + 1] - e0;
+  const int2 bb = P.base[b];
+  for (int j = threadIdx.x; j < ne; j += blockDim.x) {
+    const int4 r = owner_record(P, bb, e0 + j);
+    R x1[2], x2[2], q1[4], q2[4];
+    ld2r<SOA>(x, r.x, sx, x1);
+    ld2r<SOA>(x, r.y, sx, x2);
+    ld4r<SOA>(q, r.z, sq, q1);
+    ld4r<SOA>(q, r.w, sq, q2);
+    edge_flux(x1, x2, q1, q2, adt[r.z], adt[r.w], lf + 4 * j);
+  }
+}
+
 // Owner-compute res_calc of block b:
-//  1. one flux per edge touching the block (edges on the block boundary are
-//     evaluated by both neighbouring blocks), from global memory, into LDS;
+//  1. owner_fluxes;
 //  2. each owned cell adds its edges' fluxes to res in ascending edge order
 //     (+f where it is ecell[0], -f where it is ecell[1]), as the sequential
 //     executor does, so res is bit-identical to it.  zero_acc: res is known
 //     to hold +0.0 in every owned cell (the update before it zeroed it), so
 //     the sums start from +0.0 instead of reading it: the same bits.
 // lf: LDS for the block's fluxes, [max_e][4].
-template <bool SOA, bool C4>
+template <class R, bool SOA, bool C4>
 __device__ __forceinline__ void owner_res_block(int b, const double *__restrict x,
                                                 const double *__restrict q,
-                                                const double *__restrict adt,
-                                                double *__restrict res, const OwnerArgs &P,
-                                                int sx, int sq, double *lf,
+                                                const R *__restrict adt, R *__restrict res,
+                                                const OwnerArgs &P, int sx, int sq, R *lf,
                                                 bool zero_acc = false) {
-  const int e0 = P.elem_offs[b], ne = P.elem_offs[b + 1] - e0;
-  const int2 bb = P.base[b];
-  for (int j = threadIdx.x; j < ne; j += blockDim.x) {
-    const int4 r = owner_record(P, bb, e0 + j);
-    double x1[2], x2[2], q1[4], q2[4];
-    ld2<SOA>(x, r.x, sx, x1);
-    ld2<SOA>(x, r.y, sx, x2);
-    ld4<SOA>(q, r.z, sq, q1);
-    ld4<SOA>(q, r.w, sq, q2);
-    op2_k::res_flux(x1, x2, q1, q2, adt[r.z], adt[r.w], lf + 4 * j);
-  }
+  owner_fluxes<R, SOA>(b, x, q, adt, P, sx, sq, lf);
   __syncthreads();
   const int o0 = P.owned_offs[b], no = P.owned_offs[b + 1] - o0;
   for (int i = threadIdx.x; i < no; i += blockDim.x) {
     const int cell = P.owned[o0 + i];
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    if (!zero_acc) ld4<SOA>(res, cell, sq, acc);
+    R acc[4] = {0, 0, 0, 0};
+    if (!zero_acc) ld4r<SOA>(res, cell, sq, acc);
     if (C4) {
       const ushort4 e = P.csr4[o0 + i];
       if (e.x != 0xFFFF) owner_apply(acc, lf, e.x);
@@ -519,7 +618,7 @@ __device__ __forceinline__ void owner_res_block(int b, const double *__restrict 
       for (int k = P.csr_offs[o0 + i]; k < P.csr_offs[o0 + i + 1]; ++k)
         owner_apply(acc, lf, (int)P.csr[k]);
     }
-    st4<SOA>(res, cell, sq, acc);
+    st4r<SOA>(res, cell, sq, acc);
   }
 }
 
@@ -527,9 +626,9 @@ __device__ __forceinline__ void owner_res_block(int b, const double *__restrict 
 // fusion inside a captured step): each owned cell's fixed-width record lists
 // its interior increments, then its boundary edges as 0x8000 | j, j indexing
 // the block's list of boundary edges.  The interior fluxes are summed first,
-// in edge order, then the boundary fluxes, added by bres_calc itself into the
-// running sum in boundary-edge order: the order of res_calc then bres_calc in
-// the sequential executor, so res is bit-identical to it.
+// in edge order, then the boundary fluxes, in boundary-edge order: the order
+// of res_calc then bres_calc in the sequential executor, so res is
+// bit-identical to it.
 struct BoundaryArgs {
   const ushort4 *rec;   // per owned cell: up to four entries, 0xFFFF = none
   const int *offs;      // [nblocks+1] per block: its boundary edges' start
@@ -542,57 +641,58 @@ struct BoundaryArgs {
   const double *qinf;
 };
 
-// QI: each boundary edge with its member's free stream (B.bmesh, B.qinf),
-// else the program's qinf.
-template <bool SOA, bool QI = false>
+// Adds the entries `e` of one owned cell to acc: interior fluxes from lf,
+// boundary edges (bb0: the block's first in B.edges) evaluated here.  QI: each
+// boundary edge with its member's free stream (B.bmesh, B.qinf), else the
+// program's qinf.
+template <class R, bool SOA, bool QI>
+__device__ __forceinline__ void owner_entries(R *acc, ushort4 e, int cell, int bb0,
+                                              const double *__restrict x,
+                                              const double *__restrict q,
+                                              const R *__restrict adt, const BoundaryArgs &B,
+                                              int sx, int sq, const R *lf) {
+  const unsigned short ent[4] = {e.x, e.y, e.z, e.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (ent[k] == 0xFFFF) continue;
+    if (ent[k] & 0x8000) {
+      const int be = B.edges[bb0 + (ent[k] & 0x7FFF)];
+      const int2 bn = B.pbedge[be];
+      R x1[2], x2[2], q1[4];
+      ld2r<SOA>(x, bn.x, sx, x1);
+      ld2r<SOA>(x, bn.y, sx, x2);
+      ld4r<SOA>(q, cell, sq, q1);
+      const R a1 = adt[cell];
+      const int bnd = B.bound[be];
+      if constexpr (std::is_same<R, float>::value)
+        op2_kf::bres_calc(x1, x2, q1, &a1, acc, &bnd);
+      else if constexpr (QI)
+        op2_k::bres_calc_q(x1, x2, q1, &a1, acc, &bnd, B.qinf + 4 * (size_t)B.bmesh[be]);
+      else
+        op2_k::bres_calc(x1, x2, q1, &a1, acc, &bnd);
+    } else {
+      owner_apply(acc, lf, (int)ent[k]);
+    }
+  }
+}
+
+template <class R, bool SOA, bool QI = false>
 __device__ __forceinline__ void owner_res_bres_block(int b, const double *__restrict x,
                                                      const double *__restrict q,
-                                                     const double *__restrict adt,
-                                                     double *__restrict res,
-                                                     const OwnerArgs &P, const BoundaryArgs &B,
-                                                     int sx, int sq, double *lf,
-                                                     bool zero_acc = false) {
-  const int e0 = P.elem_offs[b], ne = P.elem_offs[b + 1] - e0;
-  const int2 bb = P.base[b];
-  for (int j = threadIdx.x; j < ne; j += blockDim.x) {
-    const int4 r = owner_record(P, bb, e0 + j);
-    double x1[2], x2[2], q1[4], q2[4];
-    ld2<SOA>(x, r.x, sx, x1);
-    ld2<SOA>(x, r.y, sx, x2);
-    ld4<SOA>(q, r.z, sq, q1);
-    ld4<SOA>(q, r.w, sq, q2);
-    op2_k::res_flux(x1, x2, q1, q2, adt[r.z], adt[r.w], lf + 4 * j);
-  }
+                                                     const R *__restrict adt,
+                                                     R *__restrict res, const OwnerArgs &P,
+                                                     const BoundaryArgs &B, int sx, int sq,
+                                                     R *lf, bool zero_acc = false) {
+  owner_fluxes<R, SOA>(b, x, q, adt, P, sx, sq, lf);
   __syncthreads();
   const int o0 = P.owned_offs[b], no = P.owned_offs[b + 1] - o0;
   const int bb0 = B.offs[b];
   for (int i = threadIdx.x; i < no; i += blockDim.x) {
     const int cell = P.owned[o0 + i];
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    if (!zero_acc) ld4<SOA>(res, cell, sq, acc);
-    const ushort4 e = B.rec[o0 + i];
-    const unsigned short ent[4] = {e.x, e.y, e.z, e.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (ent[k] == 0xFFFF) continue;
-      if (ent[k] & 0x8000) {
-        const int be = B.edges[bb0 + (ent[k] & 0x7FFF)];
-        const int2 bn = B.pbedge[be];
-        double x1[2], x2[2], q1[4];
-        ld2<SOA>(x, bn.x, sx, x1);
-        ld2<SOA>(x, bn.y, sx, x2);
-        ld4<SOA>(q, cell, sq, q1);
-        const double a1 = adt[cell];
-        const int bnd = B.bound[be];
-        if constexpr (QI)
-          op2_k::bres_calc_q(x1, x2, q1, &a1, acc, &bnd, B.qinf + 4 * (size_t)B.bmesh[be]);
-        else
-          op2_k::bres_calc(x1, x2, q1, &a1, acc, &bnd);
-      } else {
-        owner_apply(acc, lf, (int)ent[k]);
-      }
-    }
-    st4<SOA>(res, cell, sq, acc);
+    R acc[4] = {0, 0, 0, 0};
+    if (!zero_acc) ld4r<SOA>(res, cell, sq, acc);
+    owner_entries<R, SOA, QI>(acc, B.rec[o0 + i], cell, bb0, x, q, adt, B, sx, sq, lf);
+    st4r<SOA>(res, cell, sq, acc);
   }
 }
 

@@ -35,6 +35,7 @@
 #include "op2_hip_rt.h"
 #include "op2h_plan_build.h"
 #include "airfoil_device.h"
+#include "airfoil_patch.h"
 #include "op2h_reduce.h"
 
 #define KCHECK(x)                                                            \
@@ -541,14 +542,16 @@ static OwnerArgs owner_args_res(const op2h_owner_plan *p, const op_arg *args,
 }
 
 // Owner-compute res_calc (op2_dev::owner_res_block), one workgroup per block
-// of owned cells, blocks in XCD order.  LDS: fluxes [max_e][4].
-template <bool SOA, bool C4>
+// of owned cells, blocks in XCD order.  R: the type of adt and res (float:
+// mixed mode, SP fluxes from x and q rounded).  LDS: fluxes [max_e][4].
+template <class R, bool SOA, bool C4>
 __global__ void __launch_bounds__(1024)
     k_res_owner(const double *__restrict x, const double *__restrict q,
-                const double *__restrict adt, double *__restrict res,
-                OwnerArgs P, int sx, int sq, int zero_acc) {
+                const R *__restrict adt, R *__restrict res, OwnerArgs P, int sx, int sq,
+                int zero_acc) {
   extern __shared__ double lf[];
-  owner_res_block<SOA, C4>(xcd_block(kXcds), x, q, adt, res, P, sx, sq, lf, zero_acc != 0);
+  owner_res_block<R, SOA, C4>(xcd_block(kXcds), x, q, adt, res, P, sx, sq, (R *)lf,
+                              zero_acc != 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -695,32 +698,9 @@ __global__ void __launch_bounds__(1024)
 // partials visible across XCDs, so no device-scope fence is needed inside the
 // streaming kernel (on a multi-XCD gfx950 such a fence writes back L2).
 // ---------------------------------------------------------------------------
-struct MaxLoc {
-  double v;
-  int loc;
-};
-
-__device__ __forceinline__ MaxLoc maxloc_combine(MaxLoc a, MaxLoc b) {
-  // larger value wins; equal values keep the lower element index, so the
-  // result is the first element in set order reaching the maximum
-  if (b.v > a.v || (b.v == a.v && b.loc < a.loc)) return b;
-  return a;
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-__device__ __forceinline__ MaxLoc wave_maxloc(MaxLoc m) {
-  for (int o = 32; o > 0; o >>= 1) {
-    MaxLoc t;
-    t.v = __shfl_xor(m.v, o, 64);
-    t.loc = __shfl_xor(m.loc, o, 64);
-    m = maxloc_combine(m, t);
-  }
-  return m;
-}
+using op2h_red::MaxLoc;
+using op2h_red::UpdateAcc;
+using op2h_red::UpdateParts;
 
 // The cells a workgroup of the update (or of a direct chain fused with it)
 // takes, and the partial it writes: with chunk > 0 the contiguous cells
@@ -740,52 +720,30 @@ __device__ __forceinline__ CellRange cell_range(int n, int chunk) {
           (int)(gridDim.x * blockDim.x)};
 }
 
-template <bool SOA>
+// R: the type of res and adt (float: mixed mode, the update in FP64 from them).
+template <class R, bool SOA>
 __global__ void __launch_bounds__(1024)
-    k_update(const double *__restrict qold, double *__restrict q,
-             double *__restrict res, const double *__restrict adt, int n, int s,
-             double *__restrict part_sum, double *__restrict part_max,
-             int *__restrict part_loc, const int *__restrict oldidx, int chunk) {
-  __shared__ double s_sum[16];
-  __shared__ double s_max[16];
-  __shared__ int s_loc[16];
-  double rms = 0.0;
-  MaxLoc ml{-INFINITY, 0x7fffffff};
+    k_update(const double *__restrict qold, double *__restrict q, R *__restrict res,
+             const R *__restrict adt, int n, int s, UpdateParts parts,
+             const int *__restrict oldidx, int chunk) {
+  UpdateAcc acc;
   const CellRange cr = cell_range(n, chunk);
   for (int c = cr.c; c < cr.end; c += cr.step) {
-    double qo[4], qn[4], r[4], a = adt[c], mx = ml.v;
-    int loc = ml.loc;
+    double qo[4], qn[4], r[4], cs = 0.0;
+    R rr[4];
+    const double a = (double)adt[c];
     ld4<SOA>(qold, c, s, qo);
-    ld4<SOA>(res, c, s, r);
+    ld4r<SOA>(res, c, s, rr);
+    for (int d = 0; d < 4; ++d) r[d] = (double)rr[d];
     // op_arg_idx: the application's element index (transparent renumbering)
-    int ci = oldidx ? oldidx[c] : c;
-    op2_k::update(qo, qn, r, &a, &rms, &mx, &ci, &loc);
-    ml.v = mx;
-    ml.loc = loc;
+    const int ci = oldidx ? oldidx[c] : c;
+    op2_k::update(qo, qn, r, &a, &cs, &acc.ml.v, &ci, &acc.ml.loc);
+    op2h_red::sum2_add(acc.rms, cs);
     st4<SOA>(q, c, s, qn);
-    st4<SOA>(res, c, s, r);
+    const R z[4] = {0, 0, 0, 0};
+    st4r<SOA>(res, c, s, z);
   }
-  rms = wave_sum(rms);
-  ml = wave_maxloc(ml);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    s_sum[wave] = rms;
-    s_max[wave] = ml.v;
-    s_loc[wave] = ml.loc;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double bs = 0.0;
-    MaxLoc bm{-INFINITY, 0x7fffffff};
-    const int nw = (blockDim.x + 63) >> 6;
-    for (int w = 0; w < nw; ++w) {
-      bs += s_sum[w];
-      bm = maxloc_combine(bm, MaxLoc{s_max[w], s_loc[w]});
-    }
-    part_sum[cr.L] = bs;
-    part_max[cr.L] = bm.v;
-    part_loc[cr.L] = bm.loc;
-  }
+  op2h_red::write_partial(acc, parts, cr.L);
 }
 
 // Two groups of 256 threads: group 0 finishes rms (sum), group 1 maxerr and
@@ -794,18 +752,16 @@ __global__ void __launch_bounds__(1024)
 constexpr int kFinishThreads = 2 * op2h_red::kRedThreads;
 
 __global__ void __launch_bounds__(kFinishThreads)
-    k_update_finish(const double *__restrict part_sum,
-                    const double *__restrict part_max,
-                    const int *__restrict part_loc, int nparts,
-                    double *__restrict slot_rms, double *__restrict slot_max) {
-  __shared__ double s_v[2][op2h_red::kRedThreads / 64];
+    k_update_finish(UpdateParts parts, int nparts, double *__restrict slot_rms,
+                    double *__restrict slot_max) {
+  __shared__ double s_v[2][op2h_red::kRedThreads / 64], s_lo[2][op2h_red::kRedThreads / 64];
   __shared__ int s_l[2][op2h_red::kRedThreads / 64];
   const int grp = threadIdx.x / op2h_red::kRedThreads;
   const int t = threadIdx.x % op2h_red::kRedThreads;
   // one call site for both groups (the reduction holds a workgroup barrier)
-  const op2h_red::ValLoc r =
-      op2h_red::group_reduce(grp == 0 ? part_sum : part_max, grp == 0 ? nullptr : part_loc,
-                             nparts, grp == 0 ? 1 : 2, t, s_v[grp], s_l[grp]);
+  const op2h_red::ValLoc r = op2h_red::group_reduce(
+      grp == 0 ? parts.hi : parts.mx, grp == 0 ? nullptr : parts.loc,
+      grp == 0 ? parts.lo : nullptr, nparts, grp == 0 ? 4 : 2, t, s_v[grp], s_l[grp], s_lo[grp]);
   if (t == 0) {
     if (grp == 0) {
       slot_rms[0] = r.v;
@@ -822,43 +778,6 @@ __global__ void __launch_bounds__(kFinishThreads)
 // reductions stay FP64.
 // ---------------------------------------------------------------------------
 template <bool SOA>
-__device__ __forceinline__ void ld2f(const double *__restrict p, int n, int s, float *v) {
-  double t[2];
-  ld2<SOA>(p, n, s, t);
-  v[0] = (float)t[0];
-  v[1] = (float)t[1];
-}
-
-template <bool SOA>
-__device__ __forceinline__ void ld4f(const double *__restrict p, int n, int s, float *v) {
-  double t[4];
-  ld4<SOA>(p, n, s, t);
-  for (int d = 0; d < 4; ++d) v[d] = (float)t[d];
-}
-
-template <bool SOA>
-__device__ __forceinline__ void ld4s(const float *__restrict p, int n, int s, float *v) {
-  if (SOA) {
-    for (int d = 0; d < 4; ++d) v[d] = p[(size_t)d * s + n];
-  } else {
-    float4 a = *reinterpret_cast<const float4 *>(p + 4 * (size_t)n);
-    v[0] = a.x;
-    v[1] = a.y;
-    v[2] = a.z;
-    v[3] = a.w;
-  }
-}
-
-template <bool SOA>
-__device__ __forceinline__ void st4s(float *__restrict p, int n, int s, const float *v) {
-  if (SOA) {
-    for (int d = 0; d < 4; ++d) p[(size_t)d * s + n] = v[d];
-  } else {
-    *reinterpret_cast<float4 *>(p + 4 * (size_t)n) = make_float4(v[0], v[1], v[2], v[3]);
-  }
-}
-
-template <bool SOA>
 __device__ __forceinline__ void atomic_add4s(float *p, int n, int s, const float *v) {
   size_t st = SOA ? (size_t)s : 1, base = SOA ? (size_t)n : 4 * (size_t)n;
   for (int d = 0; d < 4; ++d) unsafeAtomicAdd(p + base + d * st, v[d]);
@@ -872,11 +791,11 @@ __global__ void k_adt_calc_mixed(const double *__restrict x, const double *__res
   if (c >= n) return;
   int4 cn = reinterpret_cast<const int4 *>(pcell)[c];
   float x1[2], x2[2], x3[2], x4[2], qc[4], a;
-  ld2f<SOA>(x, cn.x, sx, x1);
-  ld2f<SOA>(x, cn.y, sx, x2);
-  ld2f<SOA>(x, cn.z, sx, x3);
-  ld2f<SOA>(x, cn.w, sx, x4);
-  ld4f<SOA>(q, c, sq, qc);
+  ld2r<SOA>(x, cn.x, sx, x1);
+  ld2r<SOA>(x, cn.y, sx, x2);
+  ld2r<SOA>(x, cn.z, sx, x3);
+  ld2r<SOA>(x, cn.w, sx, x4);
+  ld4r<SOA>(q, c, sq, qc);
   op2_kf::adt_calc(x1, x2, x3, x4, qc, &a);
   adt[c] = a;
 }
@@ -890,10 +809,10 @@ __global__ void k_res_atomic_mixed(const double *__restrict x, const double *__r
   if (e >= n) return;
   int2 en = pedge[e], ec = pecell[e];
   float x1[2], x2[2], q1[4], q2[4];
-  ld2f<SOA>(x, en.x, sx, x1);
-  ld2f<SOA>(x, en.y, sx, x2);
-  ld4f<SOA>(q, ec.x, sq, q1);
-  ld4f<SOA>(q, ec.y, sq, q2);
+  ld2r<SOA>(x, en.x, sx, x1);
+  ld2r<SOA>(x, en.y, sx, x2);
+  ld4r<SOA>(q, ec.x, sq, q1);
+  ld4r<SOA>(q, ec.y, sq, q2);
   float a1 = adt[ec.x], a2 = adt[ec.y];
   float r1[4] = {0.f, 0.f, 0.f, 0.f}, r2[4] = {0.f, 0.f, 0.f, 0.f};
   op2_kf::res_calc(x1, x2, q1, q2, &a1, &a2, r1, r2);
@@ -916,10 +835,10 @@ __global__ void __launch_bounds__(1024)
   const int has = rr.x >= 0;
   if (has) {
     float x1[2], x2[2], qa[4], qb[4];
-    ld2f<SOA>(x, rr.x, sx, x1);
-    ld2f<SOA>(x, rr.y, sx, x2);
-    ld4f<SOA>(q, cell, sq, qa);
-    ld4f<SOA>(q, rr.z, sq, qb);
+    ld2r<SOA>(x, rr.x, sx, x1);
+    ld2r<SOA>(x, rr.y, sx, x2);
+    ld4r<SOA>(q, cell, sq, qa);
+    ld4r<SOA>(q, rr.z, sq, qb);
     const bool second = rr.w != 0;
     float q1[4], q2[4];
     for (int d = 0; d < 4; ++d) {
@@ -934,7 +853,7 @@ __global__ void __launch_bounds__(1024)
   }
   static_assert(K == 4, "quad broadcasts assume four lanes per cell");
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
-  if (k == 0 && valid) ld4s<SOA>(res, cell, sq, acc);
+  if (k == 0 && valid) ld4r<SOA>(res, cell, sq, acc);
   float v[4][4];
   int hv[4];
   for (int d = 0; d < 4; ++d) {
@@ -950,47 +869,7 @@ __global__ void __launch_bounds__(1024)
   for (int j = 0; j < 4; ++j)
     if (hv[j])
       for (int d = 0; d < 4; ++d) acc[d] += v[j][d];
-  if (k == 0 && valid) st4s<SOA>(res, cell, sq, acc);
-}
-
-// Mixed precision (SP fluxes, FP32 adt and res; x and q read as FP64 and
-// rounded), same structure as k_res_owner.
-template <bool SOA, bool C4>
-__global__ void __launch_bounds__(1024)
-    k_res_owner_mixed(const double *__restrict x, const double *__restrict q,
-                      const float *__restrict adt, float *__restrict res,
-                      OwnerArgs P, int sx, int sq, int zero_acc) {
-  extern __shared__ float lff[];
-  const int b = xcd_block(kXcds);
-  const int e0 = P.elem_offs[b], ne = P.elem_offs[b + 1] - e0;
-  const int2 bb = P.base[b];
-  for (int j = threadIdx.x; j < ne; j += blockDim.x) {
-    const int4 r = owner_record(P, bb, e0 + j);
-    float x1[2], x2[2], q1[4], q2[4];
-    ld2f<SOA>(x, r.x, sx, x1);
-    ld2f<SOA>(x, r.y, sx, x2);
-    ld4f<SOA>(q, r.z, sq, q1);
-    ld4f<SOA>(q, r.w, sq, q2);
-    op2_kf::res_flux(x1, x2, q1, q2, adt[r.z], adt[r.w], lff + 4 * j);
-  }
-  __syncthreads();
-  const int o0 = P.owned_offs[b], no = P.owned_offs[b + 1] - o0;
-  for (int i = threadIdx.x; i < no; i += blockDim.x) {
-    const int cell = P.owned[o0 + i];
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    if (!zero_acc) ld4s<SOA>(res, cell, sq, acc);
-    if (C4) {
-      const ushort4 e = P.csr4[o0 + i];
-      if (e.x != 0xFFFF) owner_apply(acc, lff, e.x);
-      if (e.y != 0xFFFF) owner_apply(acc, lff, e.y);
-      if (e.z != 0xFFFF) owner_apply(acc, lff, e.z);
-      if (e.w != 0xFFFF) owner_apply(acc, lff, e.w);
-    } else {
-      for (int k = P.csr_offs[o0 + i]; k < P.csr_offs[o0 + i + 1]; ++k)
-        owner_apply(acc, lff, (int)P.csr[k]);
-    }
-    st4s<SOA>(res, cell, sq, acc);
-  }
+  if (k == 0 && valid) st4r<SOA>(res, cell, sq, acc);
 }
 
 template <bool SOA>
@@ -1000,9 +879,9 @@ __device__ __forceinline__ void bres_edge_mixed(const double *__restrict x,
                                                 int cell, int bound, int sx, int sq,
                                                 float *r) {
   float x1[2], x2[2], q1[4];
-  ld2f<SOA>(x, bn.x, sx, x1);
-  ld2f<SOA>(x, bn.y, sx, x2);
-  ld4f<SOA>(q, cell, sq, q1);
+  ld2r<SOA>(x, bn.x, sx, x1);
+  ld2r<SOA>(x, bn.y, sx, x2);
+  ld4r<SOA>(q, cell, sq, q1);
   float a1 = adt[cell];
   for (int d = 0; d < 4; ++d) r[d] = 0.f;
   op2_kf::bres_calc(x1, x2, q1, &a1, r, &bound);
@@ -1035,65 +914,14 @@ __global__ void k_bres_gather_mixed(const double *__restrict x, const double *__
   if (t >= ntargets) return;
   int cell = targets[t];
   float acc[4];
-  ld4s<SOA>(res, cell, sq, acc);
+  ld4r<SOA>(res, cell, sq, acc);
   for (int k = offsets[t]; k < offsets[t + 1]; ++k) {
     int e = entries[k];
     float r[4];
     bres_edge_mixed<SOA>(x, q, adt, pbedge[e], cell, bound[e], sx, sq, r);
     for (int d = 0; d < 4; ++d) acc[d] += r[d];
   }
-  st4s<SOA>(res, cell, sq, acc);
-}
-
-template <bool SOA>
-__global__ void __launch_bounds__(1024)
-    k_update_mixed(const double *__restrict qold, double *__restrict q,
-                   float *__restrict res, const float *__restrict adt, int n, int s,
-                   double *__restrict part_sum, double *__restrict part_max,
-                   int *__restrict part_loc, const int *__restrict oldidx, int chunk) {
-  __shared__ double s_sum[16];
-  __shared__ double s_max[16];
-  __shared__ int s_loc[16];
-  double rms = 0.0;
-  MaxLoc ml{-INFINITY, 0x7fffffff};
-  const CellRange cr = cell_range(n, chunk);
-  for (int c = cr.c; c < cr.end; c += cr.step) {
-    double qo[4], qn[4], r[4], a = (double)adt[c], mx = ml.v;
-    float rf[4];
-    int loc = ml.loc;
-    ld4<SOA>(qold, c, s, qo);
-    ld4s<SOA>(res, c, s, rf);
-    for (int d = 0; d < 4; ++d) r[d] = (double)rf[d];
-    // op_arg_idx: the application's element index (transparent renumbering)
-    int ci = oldidx ? oldidx[c] : c;
-    op2_k::update(qo, qn, r, &a, &rms, &mx, &ci, &loc);
-    ml.v = mx;
-    ml.loc = loc;
-    st4<SOA>(q, c, s, qn);
-    const float z[4] = {0.f, 0.f, 0.f, 0.f};
-    st4s<SOA>(res, c, s, z);
-  }
-  rms = wave_sum(rms);
-  ml = wave_maxloc(ml);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    s_sum[wave] = rms;
-    s_max[wave] = ml.v;
-    s_loc[wave] = ml.loc;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double bs = 0.0;
-    MaxLoc bm{-INFINITY, 0x7fffffff};
-    const int nw = (blockDim.x + 63) >> 6;
-    for (int w = 0; w < nw; ++w) {
-      bs += s_sum[w];
-      bm = maxloc_combine(bm, MaxLoc{s_max[w], s_loc[w]});
-    }
-    part_sum[cr.L] = bs;
-    part_max[cr.L] = bm.v;
-    part_loc[cr.L] = bm.loc;
-  }
+  st4r<SOA>(res, cell, sq, acc);
 }
 
 }  // namespace
@@ -1143,10 +971,14 @@ void account(int kernel_idx, op_set set, int nargs, const op_arg *args) {
 //     own cell's q only);
 //   - an owner-plan res_calc is held until the bres_calc that follows and
 //     both run as one owner launch, each owned cell adding its boundary
-//     fluxes after its interior ones.
+//     fluxes after its interior ones;
+//   - whole time steps (save_soln, then twice adt_calc, res_calc, bres_calc,
+//     update) run as two launches, one per half step (k_half_step), where the
+//     owner plan covers every cell and its patches fit their lists.
 // Every cell sees the operations of the unfused loops in the same order, and
-// the update keeps its grid, block and partials, so every result is the
-// unfused one bit for bit.  Anything else flushes a pending launch as it was.
+// the reductions are sums of pairs and extrema that do not depend on how the
+// cells are grouped, so every result is the unfused one bit for bit.  Anything
+// else launches what is recorded as it was.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -1158,48 +990,33 @@ __global__ void __launch_bounds__(1024)
     k_direct_chain(const double *qold, double *__restrict q, R *__restrict res,
                    R *adt, double *qold_out, const double *__restrict x,
                    const int *__restrict pcell, const uint2 *__restrict prow,
-                   const int *__restrict pbase, int n, int s, int sx,
-                   double *__restrict part_sum, double *__restrict part_max,
-                   int *__restrict part_loc, const int *__restrict oldidx, int chunk,
-                   int res_dead) {
+                   const int *__restrict pbase, int n, int s, int sx, UpdateParts parts,
+                   const int *__restrict oldidx, int chunk, int res_dead) {
   // qold (read by update, written by save_soln) and adt (read by update,
   // written by adt_calc) are read before they are written, by the same
   // thread for the same cell: not restrict-qualified.  res_dead: the update's
   // zeros in res are not stored (the res_calc that follows in the same step
   // starts its sums from +0.0 instead of reading them)
   constexpr bool MIX = std::is_same<R, float>::value;
-  __shared__ double s_sum[16];
-  __shared__ double s_max[16];
-  __shared__ int s_loc[16];
-  double rms = 0.0;
-  MaxLoc ml{-INFINITY, 0x7fffffff};
+  UpdateAcc acc;
   // the update's cells per workgroup (its partials are the update's)
   const CellRange cr = cell_range(n, chunk);
   for (int c = cr.c; c < cr.end; c += cr.step) {
     double qn[4];
     if (UPD) {
-      double qo[4], r[4], a = (double)adt[c], mx = ml.v;
-      int loc = ml.loc;
+      double qo[4], r[4], cs = 0.0;
+      const double a = (double)adt[c];
+      R rr[4];
       ld4<SOA>(qold, c, s, qo);
-      if constexpr (MIX) {
-        float rf[4];
-        ld4s<SOA>(res, c, s, rf);
-        for (int d = 0; d < 4; ++d) r[d] = (double)rf[d];
-      } else {
-        ld4<SOA>(res, c, s, r);
-      }
-      int ci = oldidx ? oldidx[c] : c;
-      op2_k::update(qo, qn, r, &a, &rms, &mx, &ci, &loc);
-      ml.v = mx;
-      ml.loc = loc;
+      ld4r<SOA>(res, c, s, rr);
+      for (int d = 0; d < 4; ++d) r[d] = (double)rr[d];
+      const int ci = oldidx ? oldidx[c] : c;
+      op2_k::update(qo, qn, r, &a, &cs, &acc.ml.v, &ci, &acc.ml.loc);
+      op2h_red::sum2_add(acc.rms, cs);
       st4<SOA>(q, c, s, qn);
       if (!res_dead) {
-        if constexpr (MIX) {
-          const float z[4] = {0.f, 0.f, 0.f, 0.f};
-          st4s<SOA>(res, c, s, z);
-        } else {
-          st4<SOA>(res, c, s, r);
-        }
+        const R z[4] = {0, 0, 0, 0};
+        st4r<SOA>(res, c, s, z);
       }
     } else {
       ld4<SOA>(q, c, s, qn);
@@ -1214,57 +1031,70 @@ __global__ void __launch_bounds__(1024)
     } else {
       cn = reinterpret_cast<const int4 *>(pcell)[c];
     }
-    if constexpr (MIX) {
-      float x1[2], x2[2], x3[2], x4[2], qf[4], a2;
-      ld2f<SOA>(x, cn.x, sx, x1);
-      ld2f<SOA>(x, cn.y, sx, x2);
-      ld2f<SOA>(x, cn.z, sx, x3);
-      ld2f<SOA>(x, cn.w, sx, x4);
-      for (int d = 0; d < 4; ++d) qf[d] = (float)qn[d];
-      op2_kf::adt_calc(x1, x2, x3, x4, qf, &a2);
-      adt[c] = a2;
-    } else {
-      double x1[2], x2[2], x3[2], x4[2], a2;
-      ld2<SOA>(x, cn.x, sx, x1);
-      ld2<SOA>(x, cn.y, sx, x2);
-      ld2<SOA>(x, cn.z, sx, x3);
-      ld2<SOA>(x, cn.w, sx, x4);
-      op2_k::adt_calc(x1, x2, x3, x4, qn, &a2);
-      adt[c] = a2;
-    }
+    R x1[2], x2[2], x3[2], x4[2], qr[4] = {(R)qn[0], (R)qn[1], (R)qn[2], (R)qn[3]}, a2;
+    ld2r<SOA>(x, cn.x, sx, x1);
+    ld2r<SOA>(x, cn.y, sx, x2);
+    ld2r<SOA>(x, cn.z, sx, x3);
+    ld2r<SOA>(x, cn.w, sx, x4);
+    if constexpr (MIX)
+      op2_kf::adt_calc(x1, x2, x3, x4, qr, &a2);
+    else
+      op2_k::adt_calc(x1, x2, x3, x4, qr, &a2);
+    adt[c] = a2;
   }
-  if (!UPD) return;
-  // the partials of k_update, by the same tree
-  rms = wave_sum(rms);
-  ml = wave_maxloc(ml);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    s_sum[wave] = rms;
-    s_max[wave] = ml.v;
-    s_loc[wave] = ml.loc;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double bsum = 0.0;
-    MaxLoc bm{-INFINITY, 0x7fffffff};
-    const int nw = (blockDim.x + 63) >> 6;
-    for (int w = 0; w < nw; ++w) {
-      bsum += s_sum[w];
-      bm = maxloc_combine(bm, MaxLoc{s_max[w], s_loc[w]});
-    }
-    part_sum[cr.L] = bsum;
-    part_max[cr.L] = bm.v;
-    part_loc[cr.L] = bm.loc;
-  }
+  if (UPD) op2h_red::write_partial(acc, parts, cr.L);
 }
 
-template <bool SOA>
+template <class R, bool SOA>
 __global__ void __launch_bounds__(1024)
     k_res_bres_owner(const double *__restrict x, const double *__restrict q,
-                     const double *__restrict adt, double *__restrict res, OwnerArgs P,
-                     BoundaryArgs B, int sx, int sq, int zero_acc) {
+                     const R *__restrict adt, R *__restrict res, OwnerArgs P, BoundaryArgs B,
+                     int sx, int sq, int zero_acc) {
   extern __shared__ double lf[];
-  owner_res_bres_block<SOA>(xcd_block(kXcds), x, q, adt, res, P, B, sx, sq, lf, zero_acc != 0);
+  owner_res_bres_block<R, SOA>(xcd_block(kXcds), x, q, adt, res, P, B, sx, sq, (R *)lf,
+                               zero_acc != 0);
+}
+
+// One half step (op2_dev::half_step_patch) over all patches of the owner
+// plan: a grid of workgroups that walk them, with one reduction partial per
+// workgroup.
+template <class R, bool SOA>
+__global__ void __launch_bounds__(1024)
+    k_half_step(HalfArgs<R> H, PatchArgs P, BoundaryArgs B, int npatch, int nc, int nn,
+                UpdateParts parts) {
+  extern __shared__ double lf[];
+  UpdateAcc acc;
+  for (int b = xcd_block(kXcds); b < npatch; b += gridDim.x) {
+    half_step_patch<R, SOA, false>(b, H, P, B, 0, lf, nc, nn, acc);
+    __syncthreads();  // the next patch restages the LDS
+  }
+  op2h_red::write_partial(acc, parts, blockIdx.x);
+}
+
+// Rows of a four-node map as 16-bit offsets from the lowest node of their
+// 64-cell group, one wave per group; *wide is set where a group's nodes span
+// more than 65535.
+__global__ void __launch_bounds__(256)
+    k_pack_rows(const int4 *__restrict pcell, int n, uint2 *__restrict rec,
+                int *__restrict base, int *wide) {
+  const int g = blockIdx.x * 4 + (threadIdx.x >> 6), c = 64 * g + (threadIdx.x & 63);
+  if (64 * g >= n) return;  // the whole wave
+  const bool in = c < n;
+  const int4 r = in ? pcell[c] : make_int4(INT_MAX, INT_MAX, INT_MAX, INT_MAX);
+  int lo = min(min(r.x, r.y), min(r.z, r.w));
+  int hi = in ? max(max(r.x, r.y), max(r.z, r.w)) : -1;
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o));
+    hi = max(hi, __shfl_xor(hi, o));
+  }
+  if (hi - lo > 0xFFFF) {
+    *wide = 1;
+    return;
+  }
+  if ((threadIdx.x & 63) == 0) base[g] = lo;
+  if (in)
+    rec[c] = make_uint2((unsigned)(r.x - lo) | ((unsigned)(r.y - lo) << 16),
+                        (unsigned)(r.z - lo) | ((unsigned)(r.w - lo) << 16));
 }
 
 // A pending run of direct loops over one cell set: [update] [save_soln].
@@ -1285,112 +1115,316 @@ UpdateShape update_shape(int n, int bs) {
   return {std::max(1, std::min(grid_for(n, bs), 2048)), 0};
 }
 
+// One {hi, lo, max, loc} partial per workgroup in `mem` (g of them).
+constexpr size_t kPartBytes = 3 * sizeof(double) + sizeof(int);
+UpdateParts update_parts(void *mem, int g) {
+  double *d = (double *)mem;
+  return UpdateParts{d, d + g, d + 2 * (size_t)g, (int *)(d + 3 * (size_t)g)};
+}
+
+// Most workgroups of a half step: the partials one reduction takes.
+constexpr int kHalfGrid = op2h_red::kRedThreads * op2h_red::kRedMaxLoads;
+
 struct PendingDirect {
   bool upd = false, save = false, soa = false;
   op_set set = nullptr;
   hipStream_t st = nullptr;
   int n = 0, s = 0;
-  // update (its partials handed to the graph's history kernel)
-  int g = 0, bs = 0, chunk = 0;
-  bool mixed = false;  // res and adt FP32 (res_f, adt_f), else FP64 (res, adt)
+  // update (its partials handed to the graph's history kernel: up to `cap`)
+  int g = 0, bs = 0, chunk = 0, cap = 0;
+  bool mixed = false;  // res and adt FP32, else FP64
   const double *qold = nullptr;
-  double *q = nullptr, *res = nullptr, *adt = nullptr;
-  float *res_f = nullptr, *adt_f = nullptr;
-  double *part_sum = nullptr, *part_max = nullptr;
-  int *part_loc = nullptr;
+  double *q = nullptr;
+  void *res = nullptr, *adt = nullptr;
+  UpdateParts parts{};
   const int *oldidx = nullptr;
   // save_soln: src -> dst, n2 16-byte vectors when run on its own
   const double *save_src = nullptr;
   double *save_dst = nullptr;
   int save_n2 = 0, save_bs = 256;
 };
-PendingDirect g_direct;
 
-void flush_direct(void *) {
-  PendingDirect P = g_direct;
-  g_direct = PendingDirect();
-  if (P.upd && P.mixed)
-    launch_k(false, nullptr, nullptr, P.soa ? k_update_mixed<true> : k_update_mixed<false>, P.g,
-             P.bs, 0, P.st, P.qold, P.q, P.res_f, (const float *)P.adt_f, P.n, P.s, P.part_sum,
-             P.part_max, P.part_loc, P.oldidx, P.chunk);
-  else if (P.upd)
-    launch_k(false, nullptr, nullptr, P.soa ? k_update<true> : k_update<false>, P.g, P.bs, 0,
-             P.st, P.qold, P.q, P.res, (const double *)P.adt, P.n, P.s, P.part_sum,
-             P.part_max, P.part_loc, P.oldidx, P.chunk);
+template <class R>
+void launch_update(bool ext, void *e0, void *e1, const PendingDirect &P) {
+  launch_k(ext, e0, e1, P.soa ? k_update<R, true> : k_update<R, false>, P.g, P.bs, 0, P.st,
+           P.qold, P.q, (R *)P.res, (const R *)P.adt, P.n, P.s, P.parts, P.oldidx, P.chunk);
+}
+
+void launch_direct(const PendingDirect &P) {
+  if (P.upd) {
+    op2h_gbl_partials_used(P.parts.hi, P.g);
+    op2h_gbl_partials_used(P.parts.mx, P.g);
+    if (P.mixed) launch_update<float>(false, nullptr, nullptr, P);
+    else launch_update<double>(false, nullptr, nullptr, P);
+  }
   if (P.save)
     launch_k(false, nullptr, nullptr, k_save_soln, grid_for(P.save_n2, P.save_bs), P.save_bs, 0,
              P.st, (const double2 *)P.save_src, (double2 *)P.save_dst, P.save_n2);
 }
 
 // A pending fused direct chain ([update] [save_soln] adt_calc per cell).
-template <class R>
-using ChainKernel = void (*)(const double *, double *, R *, R *, double *, const double *,
-                             const int *, const uint2 *, const int *, int, int, int, double *,
-                             double *, int *, const int *, int, int);
 struct PendingChain {
-  ChainKernel<double> kern = nullptr;  // FP64 res and adt
-  ChainKernel<float> kern_f = nullptr;  // mixed mode
-  float *adt_f = nullptr;
+  bool mixed = false;
   PendingDirect P;
   int g = 0, bs = 0, chunk = 0, n = 0, sq = 0, sx = 0;
-  double *q = nullptr, *adt = nullptr;
+  double *q = nullptr;
+  void *adt = nullptr;
   const double *x = nullptr;
   const int *pcell = nullptr;
   const uint2 *prow = nullptr;  // compact rows of pcell, or null
   const int *pbase = nullptr;
   hipStream_t st = nullptr;
 };
-PendingChain g_chain;
+
+template <class R>
+void launch_chain_as(const PendingChain &C, bool res_dead) {
+  const PendingDirect &P = C.P;
+  auto kern = P.upd ? (P.save ? (P.soa ? k_direct_chain<R, true, true, true> : k_direct_chain<R, false, true, true>)
+                              : (P.soa ? k_direct_chain<R, true, true, false> : k_direct_chain<R, false, true, false>))
+                    : (P.soa ? k_direct_chain<R, true, false, true> : k_direct_chain<R, false, false, true>);
+  launch_k(false, nullptr, nullptr, kern, C.g, C.bs, 0, C.st, P.qold, C.q, (R *)P.res,
+           (R *)C.adt, P.save_dst, C.x, C.pcell, C.prow, C.pbase, C.n, C.sq, C.sx, P.parts,
+           P.oldidx, C.chunk, (int)(res_dead && P.upd));
+}
 
 // res_dead: the update's zeros in res are not stored (the owner res_calc
 // launched right after it sums from +0.0 over every cell of the set)
-void launch_chain(bool res_dead) {
-  const PendingChain C = g_chain;
-  g_chain = PendingChain();
-  const PendingDirect &P = C.P;
-  if (C.kern_f)
-    launch_k(false, nullptr, nullptr, C.kern_f, C.g, C.bs, 0, C.st, P.qold, C.q, P.res_f,
-             C.adt_f, P.save_dst, C.x, C.pcell, C.prow, C.pbase, C.n, C.sq, C.sx, P.part_sum,
-             P.part_max, P.part_loc, P.oldidx, C.chunk, (int)(res_dead && P.upd));
-  else
-    launch_k(false, nullptr, nullptr, C.kern, C.g, C.bs, 0, C.st, P.qold, C.q, P.res, C.adt,
-             P.save_dst, C.x, C.pcell, C.prow, C.pbase, C.n, C.sq, C.sx, P.part_sum,
-             P.part_max, P.part_loc, P.oldidx, C.chunk, (int)(res_dead && P.upd));
-  KCHECK(hipGetLastError());
+void launch_chain(const PendingChain &C, bool res_dead) {
+  if (C.P.upd) {
+    op2h_gbl_partials_used(C.P.parts.hi, C.P.g);
+    op2h_gbl_partials_used(C.P.parts.mx, C.P.g);
+  }
+  if (C.mixed) launch_chain_as<float>(C, res_dead);
+  else launch_chain_as<double>(C, res_dead);
 }
 
-void flush_chain(void *) { launch_chain(false); }
-
-// A pending owner-plan res_calc.
+// An owner-plan res_calc.
 struct PendingRes {
-  bool soa = false;
+  bool soa = false, mixed = false;
   hipStream_t st = nullptr;
   const op2h_owner_plan *plan = nullptr;
+  unsigned epoch = 0;  // op2h_plan_epoch(): the plan pointer's validity
   OwnerArgs A{};
-  const double *x = nullptr, *q = nullptr, *adt = nullptr;
-  double *res = nullptr;
+  const double *x = nullptr, *q = nullptr;
+  const void *adt = nullptr;
+  void *res = nullptr;
   int sx = 0, sq = 0, bs = 0;
   size_t lds = 0;
   op_map pecell = nullptr;
+  op_set cells = nullptr;
   bool zero = false;  // res holds the update's zeros: sums start from +0.0
 };
+
+template <class R>
+void launch_res_as(bool ext, void *e0, void *e1, const PendingRes &P) {
+  if (P.plan->nblocks)
+    launch_k(ext, e0, e1,
+             P.A.csr4 ? (P.soa ? k_res_owner<R, true, true> : k_res_owner<R, false, true>)
+                      : (P.soa ? k_res_owner<R, true, false> : k_res_owner<R, false, false>),
+             P.plan->nblocks, P.bs, P.lds, P.st, P.x, P.q, (const R *)P.adt, (R *)P.res, P.A,
+             P.sx, P.sq, (int)P.zero);
+}
+
+void launch_res(bool ext, void *e0, void *e1, const PendingRes &P) {
+  if (P.mixed) launch_res_as<float>(ext, e0, e1, P);
+  else launch_res_as<double>(ext, e0, e1, P);
+}
+
+template <class R>
+void launch_res_bres_as(const PendingRes &P, const BoundaryArgs &B) {
+  if (P.plan->nblocks)
+    launch_k(false, nullptr, nullptr, P.soa ? k_res_bres_owner<R, true> : k_res_bres_owner<R, false>,
+             P.plan->nblocks, P.bs, P.lds, P.st, P.x, P.q, (const R *)P.adt, (R *)P.res, P.A, B,
+             P.sx, P.sq, (int)P.zero);
+}
+
+// The captured loops not launched yet.  Nothing runs while a graph is being
+// captured, so the stubs only record what they would launch and the whole run
+// of loops is launched when something else comes (or the capture ends), with
+// every following loop known: g_halves, the complete [chain] res_calc
+// bres_calc groups; then at most one of g_direct ([update] [save_soln]),
+// g_chain (the same with the adt_calc that follows) or g_chain with g_res.
+struct Half {
+  bool chained = false;  // C precedes R
+  PendingChain C;
+  PendingRes R;
+  BoundaryArgs B{};
+};
+std::vector<Half> g_halves;
+PendingDirect g_direct;
+PendingChain g_chain;
+bool g_res_chained = false;  // g_chain precedes g_res
 PendingRes g_res;
 PendingRes g_last_res;  // the latest owner-plan res_calc, pending or not
 
-void launch_res_owner(const PendingRes &P) {
-  if (P.plan->nblocks)
-    launch_k(false, nullptr, nullptr,
-             P.A.csr4 ? (P.soa ? k_res_owner<true, true> : k_res_owner<false, true>)
-                      : (P.soa ? k_res_owner<true, false> : k_res_owner<false, false>),
-             P.plan->nblocks, P.bs, P.lds, P.st, P.x, P.q, P.adt, P.res, P.A, P.sx, P.sq,
-             (int)P.zero);
+// Device memory of the fused half steps for one owner plan and its dats: the
+// other copies of q and adt and the patches' lists (allocated before
+// a capture starts, for the latest owner-plan res_calc).
+struct HalfMem {
+  unsigned epoch = 0;
+  const op2h_owner_plan *plan = nullptr;
+  const double *q = nullptr;
+  bool mixed = false;
+  const int *pcell = nullptr;
+  const ushort4 *rec = nullptr;  // the boundary records the lists hold
+  double *q2 = nullptr;
+  void *adt2 = nullptr;
+  PatchArgs patches{};
+  int nc = 0, nn = 0;
+};
+HalfMem g_half_mem;
+
+// Whether halves h and k (with the direct loops D that follow k, and its
+// adt_calc C if that follows too) are one time step of the form
+//   save_soln adt_calc res_calc bres_calc update
+//             adt_calc res_calc bres_calc update [save_soln] [adt_calc]
+// on the same dats, which two k_half_step launches run.
+bool is_step(const Half &h, const Half &k, const PendingDirect *D, const PendingChain *C) {
+  const HalfMem &M = g_half_mem;
+  const PendingRes &R = h.R;
+  if (!h.chained || !k.chained || !D || !D->upd || M.epoch != op2h_plan_epoch() ||
+      R.epoch != M.epoch || M.plan != R.plan || M.q != R.q || M.mixed != R.mixed ||
+      M.pcell != h.C.pcell || M.rec != h.B.rec)
+    return false;
+  const op2h_owner_plan *p = R.plan;
+  if (!p->nblocks || p->n_owned != R.cells->size || p->max_owned > R.bs) return false;
+  const PendingRes &S = k.R;
+  if (S.plan != p || S.x != R.x || S.q != R.q || S.adt != R.adt || S.res != R.res ||
+      S.mixed != R.mixed || S.soa != R.soa || S.sx != R.sx || S.sq != R.sq || S.bs != R.bs ||
+      S.st != R.st || k.B.rec != h.B.rec || k.B.pbedge != h.B.pbedge || k.B.bound != h.B.bound)
+    return false;
+  auto chain_fits = [&](const PendingChain &c) {
+    return c.q == R.q && c.adt == R.adt && c.x == R.x && c.mixed == R.mixed &&
+           c.P.soa == R.soa && c.n == R.cells->size && c.pcell == h.C.pcell && c.st == R.st;
+  };
+  const PendingDirect &A = h.C.P, &U = k.C.P;
+  auto update_fits = [&](const PendingDirect &d) {
+    return d.upd && d.q == R.q && d.qold == A.save_dst && d.res == R.res && d.adt == R.adt &&
+           d.mixed == R.mixed && d.soa == R.soa && d.set == R.cells && d.st == R.st &&
+           d.cap >= 1 && d.oldidx == U.oldidx;
+  };
+  return A.save && A.save_src == R.q && A.save_dst != R.q && chain_fits(h.C) &&
+         chain_fits(k.C) && (!C || chain_fits(*C)) && update_fits(U) && !U.save &&
+         update_fits(*D) && (!D->save || (D->save_src == R.q && D->save_dst == A.save_dst));
 }
 
-void flush_res(void *) {
-  PendingRes P = g_res;
-  g_res = PendingRes();
-  launch_res_owner(P);
+template <class R>
+void launch_half_as(const Half &h, const HalfArgs<R> &H, const PendingDirect &D) {
+  const PendingRes &P = h.R;
+  const HalfMem &M = g_half_mem;
+  auto kern = P.soa ? k_half_step<R, true> : k_half_step<R, false>;
+  const size_t lds = patch_lds_bytes<R>(M.nc, M.nn);
+  // as many workgroups as the GPU holds at once, each walking the same number
+  // of patches: 126 us at 2.88 million cells with the 4 per CU that fit,
+  // 159 with 5 and 140 with 6 per CU (a second, nearly empty round), 125 with a
+  // quarter of the patches each; nothing in it at 720,000 (34 to 35 us)
+  int resident = 0, cus = 0, dev = 0;
+  KCHECK(hipGetDevice(&dev));
+  KCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  KCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, (const void *)kern, P.bs, lds));
+  const int npatch = P.plan->nblocks;
+  const int rounds = (npatch + std::max(1, resident * cus) - 1) / std::max(1, resident * cus);
+  const int grid = std::min((npatch + rounds - 1) / rounds, D.cap);
+  op2h_gbl_partials_used(D.parts.hi, grid);
+  op2h_gbl_partials_used(D.parts.mx, grid);
+  launch_k(false, nullptr, nullptr, kern, grid, P.bs, lds, P.st, H, M.patches, h.B, npatch, M.nc,
+           M.nn, D.parts);
 }
+
+// The time step of halves h and k as two launches (is_step holds).  D: the
+// second update; adt: an adt_calc follows it; dead_save: the next time step is
+// run the same way, so nothing reads the copy of q that D's save_soln would
+// make, nor was this step's own copy made when saved is false; zeroed: res
+// holds zeros in memory.
+template <class R>
+void launch_step_as(const Half &h, const Half &k, const PendingDirect &D, bool adt,
+                    bool dead_save, bool saved, bool zeroed) {
+  const HalfMem &M = g_half_mem;
+  double *q = const_cast<double *>(h.R.q), *qold = h.C.P.save_dst;
+  R *a = (R *)const_cast<void *>(h.R.adt), *a2 = (R *)M.adt2;
+  HalfArgs<R> H;
+  H.x = h.R.x;
+  H.q = q;
+  H.adt = a;
+  H.res = (R *)h.R.res;
+  H.qold = nullptr;  // the step's first q, which save_soln copies: q itself
+  H.q_out = M.q2;
+  H.adt_out = a2;
+  H.qold_out = qold;
+  H.oldidx = k.C.P.oldidx;
+  H.sx = h.R.sx;
+  H.sq = h.R.sq;
+  H.flags = kHalfAdt | (zeroed ? 0 : kHalfReadRes | kHalfZeroRes);
+  launch_half_as<R>(h, H, k.C.P);
+  H.q = M.q2;
+  H.adt = a2;
+  H.qold = q;
+  H.q_out = q;
+  H.adt_out = a;
+  H.flags = (adt ? kHalfAdt : kHalfCopyAdt) |
+            (D.save ? (dead_save ? 0 : kHalfSaveNew) : (saved ? 0 : kHalfSaveOld));
+  launch_half_as<R>(k, H, D);
+}
+
+// Launches everything recorded, in order: time steps as pairs of half steps,
+// other loops as direct chains and res_calc + bres_calc.
+void launch_recorded(bool direct, bool chain, bool res) {
+  const std::vector<Half> hs = std::move(g_halves);
+  g_halves.clear();
+  const PendingDirect D = g_direct;
+  const PendingChain C = g_chain;
+  const int n = (int)hs.size();
+  const bool tail_chain = chain || (res && g_res_chained);
+  // what follows half i: its update's record, and the chain's when adt_calc does too
+  auto follows = [&](int i, const PendingDirect **d, const PendingChain **c) {
+    *c = i + 1 < n ? (hs[i + 1].chained ? &hs[i + 1].C : nullptr) : tail_chain ? &C : nullptr;
+    *d = *c ? &(*c)->P : (i + 1 == n && direct) ? &D : nullptr;
+  };
+  auto step_at = [&](int i) {
+    if (i + 1 >= n) return false;
+    const PendingDirect *d;
+    const PendingChain *c;
+    follows(i + 1, &d, &c);
+    return is_step(hs[i], hs[i + 1], d, c);
+  };
+  bool folded = false;   // the chain or update after the last launch is part of it
+  bool saved = true;     // qold holds the copy of q that half i's chain makes
+  for (int i = 0; i < n;) {
+    if (step_at(i)) {
+      if (!folded) launch_chain(hs[i].C, false);
+      const bool zeroed = folded || hs[i].C.P.upd;
+      const PendingDirect *d;
+      const PendingChain *c;
+      follows(i + 1, &d, &c);
+      const bool dead = c && d->save && step_at(i + 2);
+      if (hs[i].R.mixed) launch_step_as<float>(hs[i], hs[i + 1], *d, c, dead, saved, zeroed);
+      else launch_step_as<double>(hs[i], hs[i + 1], *d, c, dead, saved, zeroed);
+      folded = true;
+      saved = !dead;
+      i += 2;
+    } else {
+      if (hs[i].chained && !folded) launch_chain(hs[i].C, hs[i].R.zero);
+      if (hs[i].R.mixed) launch_res_bres_as<float>(hs[i].R, hs[i].B);
+      else launch_res_bres_as<double>(hs[i].R, hs[i].B);
+      folded = false;
+      saved = true;
+      ++i;
+    }
+  }
+  if (direct && !folded) launch_direct(D);
+  if (tail_chain && !folded) launch_chain(C, res && g_res.zero);
+  if (res) launch_res(false, nullptr, nullptr, g_res);
+  g_direct = PendingDirect();
+  g_chain = PendingChain();
+  g_res_chained = false;
+  g_res = PendingRes();
+  KCHECK(hipGetLastError());
+}
+
+void flush_direct(void *) { launch_recorded(true, false, false); }
+void flush_chain(void *) { launch_recorded(false, true, false); }
+void flush_res(void *) { launch_recorded(false, false, true); }
+void flush_halves(void *) { launch_recorded(false, false, false); }
 
 // The fused res_calc + bres_calc records for an owner plan and the boundary
 // map (bedge -> cell), built on the host once per plan: each owned cell's
@@ -1488,60 +1522,107 @@ const BoundaryArgs *boundary_args(const op2h_owner_plan *p, op_map pbecell, op_m
 // Compact rows of a four-node map (cells -> nodes) for the fused direct
 // chain: per cell its nodes as 16-bit offsets from the lowest node of its
 // 64-cell group, 8 bytes instead of 16, where every group's nodes lie within
-// 65535 of that base (a locally numbered mesh; else null).  `build` false:
-// only a record built before (inside a capture nothing may be uploaded).
+// 65535 of that base (a locally numbered mesh; else null).  Packed on the
+// device when a capture starts: only captured chains read them, and nothing
+// may be allocated once it has started.
 struct CompactRows {
-  const uint2 *rec = nullptr;
+  unsigned epoch = 0;
+  const int *map = nullptr;
+  const uint2 *rec = nullptr;  // null: the rows do not fit
   const int *base = nullptr;
 };
+CompactRows g_rows;
+struct {
+  unsigned epoch = 0;
+  op_map map = nullptr;
+  hipStream_t st = nullptr;
+} g_last_pcell;  // the latest adt_calc's
+struct {
+  unsigned epoch = 0;
+  const op2h_owner_plan *plan = nullptr;
+  const ushort4 *rec = nullptr;
+} g_last_bres;  // the latest fused res_calc + bres_calc records built
 
-const CompactRows *compact_rows(op_map m, hipStream_t st, bool build) {
-  struct Slot {
-    unsigned epoch = 0;
-    bool ok = false;
-    CompactRows R;
-  };
-  static std::map<int, Slot> cache;
-  auto it = cache.find(m->index);
-  if (it != cache.end() && it->second.epoch == op2h_plan_epoch())
-    return it->second.ok ? &it->second.R : nullptr;
-  if (!build) return nullptr;
-  Slot &slot = cache[m->index];
-  slot = Slot();
-  slot.epoch = op2h_plan_epoch();
+const CompactRows *compact_rows(op_map m) {
+  return g_rows.epoch == op2h_plan_epoch() && g_rows.map == m->map_d && g_rows.rec ? &g_rows
+                                                                                    : nullptr;
+}
+
+void pack_compact_rows(op_map m, hipStream_t st) {
+  if (g_rows.epoch == op2h_plan_epoch() && g_rows.map == m->map_d) return;
+  g_rows = CompactRows();
+  g_rows.epoch = op2h_plan_epoch();
+  g_rows.map = m->map_d;
   const int n = m->from->size, ng = (n + 63) / 64;
-  if (m->dim != 4 || n < 1) return nullptr;
-  const int *hm = op2h::host_map(m);  // in the device numbering
-  std::vector<uint2> rec(n);
-  std::vector<int> base(ng);
-  for (int g = 0; g < ng; ++g) {
-    const int c0 = 64 * g, c1 = std::min(n, c0 + 64);
-    int lo = INT_MAX, hi = INT_MIN;
-    for (size_t i = 4 * (size_t)c0; i < 4 * (size_t)c1; ++i) {
-      lo = std::min(lo, hm[i]);
-      hi = std::max(hi, hm[i]);
-    }
-    if ((long long)hi - lo > 0xFFFF) return nullptr;
-    base[g] = lo;
-    for (int c = c0; c < c1; ++c) {
-      const int *r = hm + 4 * (size_t)c;
-      rec[c] = make_uint2((unsigned)(r[0] - lo) | ((unsigned)(r[1] - lo) << 16),
-                          (unsigned)(r[2] - lo) | ((unsigned)(r[3] - lo) << 16));
-    }
-  }
+  if (m->dim != 4 || n < 1) return;
   char name[64];
   snprintf(name, sizeof name, "compact_rows.%d", m->index);
   const size_t b_rec = (8 * (size_t)n + 255) / 256 * 256;
+  const size_t b_base = (4 * (size_t)ng + 255) / 256 * 256;
   int fresh = 0;
-  char *buf = (char *)op2h_plan_user(name, b_rec + 4 * (size_t)ng, &fresh);
-  KCHECK(hipMemcpyAsync(buf, rec.data(), 8 * (size_t)n, hipMemcpyHostToDevice, st));
-  KCHECK(hipMemcpyAsync(buf + b_rec, base.data(), 4 * (size_t)ng, hipMemcpyHostToDevice, st));
-  KCHECK(hipStreamSynchronize(st));  // rec and base are locals
-  slot.R.rec = (const uint2 *)buf;
-  slot.R.base = (const int *)(buf + b_rec);
-  slot.ok = true;
-  return &slot.R;
+  char *buf = (char *)op2h_plan_user(name, b_rec + b_base + 4, &fresh);
+  int *wide = (int *)(buf + b_rec + b_base);
+  const int zero = 0;
+  int any = 0;
+  KCHECK(hipMemcpyAsync(wide, &zero, sizeof zero, hipMemcpyHostToDevice, st));
+  k_pack_rows<<<grid_for(ng, 4), 256, 0, st>>>((const int4 *)m->map_d, n, (uint2 *)buf,
+                                               (int *)(buf + b_rec), wide);
+  KCHECK(hipMemcpyAsync(&any, wide, sizeof any, hipMemcpyDeviceToHost, st));
+  KCHECK(hipStreamSynchronize(st));
+  if (any) return;
+  g_rows.rec = (const uint2 *)buf;
+  g_rows.base = (const int *)(buf + b_rec);
 }
+
+// The memory of the fused half steps, for the latest owner-plan res_calc and
+// the latest adt_calc's map when they are over the same cells.
+void make_half_mem() {
+  const PendingRes &R = g_last_res;
+  const op_map pcell = g_last_pcell.map;
+  const unsigned now = op2h_plan_epoch();
+  g_half_mem = HalfMem();
+  if (!R.plan || R.epoch != now || g_last_pcell.epoch != now || !pcell ||
+      pcell->from != R.cells || pcell->dim != 4 || !R.plan->csr4 || !R.plan->nblocks ||
+      R.plan->n_owned != R.cells->size || R.plan->max_owned > R.bs)
+    return;
+  const op2h_owner_plan *p = R.plan;
+  if (g_last_bres.epoch != now || g_last_bres.plan != p) return;
+  char name[96];
+  int fresh = 0, part = 0;
+  HalfMem M;
+  if (!build_patches(
+          R.A, p->nblocks, g_last_bres.rec, (const int4 *)pcell->map_d, R.cells->size, R.st,
+          [&](size_t bytes) {
+            snprintf(name, sizeof name, "half_step.lists%d.%p", part++, (const void *)p);
+            return op2h_plan_user(name, bytes, &fresh);
+          },
+          &M.patches, &M.nc, &M.nn) ||
+      patch_lds_bytes<double>(M.nc, M.nn) > 64 * 1024)
+    return;
+  const size_t rows = (size_t)(R.soa ? R.cells->stride : R.cells->size);
+  const size_t b_q = 4 * sizeof(double) * rows;
+  snprintf(name, sizeof name, "half_step.q.%p", (const void *)p);
+  M.q2 = (double *)op2h_plan_user(
+      name, b_q + (R.mixed ? sizeof(float) : sizeof(double)) * rows, &fresh);
+  M.adt2 = (char *)M.q2 + b_q;
+  M.epoch = now;
+  M.plan = p;
+  M.q = R.q;
+  M.mixed = R.mixed;
+  M.pcell = pcell->map_d;
+  M.rec = g_last_bres.rec;
+  g_half_mem = M;
+}
+
+void before_capture() {
+  if (g_last_pcell.map && g_last_pcell.epoch == op2h_plan_epoch())
+    pack_compact_rows(g_last_pcell.map, g_last_pcell.st);
+  make_half_mem();
+}
+
+const struct CaptureHook {
+  CaptureHook() { op2h_register_capture_hook(before_capture); }
+} g_capture_hook;
 
 }  // namespace
 
@@ -1629,8 +1710,7 @@ extern "C" void op_par_loop_airfoil_2_adt_calc(char const *name, op_set set,
       const double *qsrc = P.upd ? P.q : P.save_src;
       const bool mixed = is_float(args[5]);
       if (P.set == set && P.soa == soa && (soa ? sq == P.s : true) && qsrc == q &&
-          (!P.upd || (P.mixed == mixed &&
-                      (mixed ? (void *)P.adt_f == args[5].data_d : P.adt == adt)))) {
+          (!P.upd || (P.mixed == mixed && P.adt == args[5].data_d))) {
         g_direct = PendingDirect();
         // [update] [save_soln] adt_calc per cell: the update's launch shape
         // (its partials), else adt_calc's
@@ -1638,25 +1718,16 @@ extern "C" void op_par_loop_airfoil_2_adt_calc(char const *name, op_set set,
         const int chunk = P.upd ? P.chunk : 0;
         PendingChain &C = g_chain;
         C = PendingChain();
-        if (mixed) {
-          C.kern_f = P.upd ? (P.save ? (soa ? k_direct_chain<float, true, true, true> : k_direct_chain<float, false, true, true>)
-                                     : (soa ? k_direct_chain<float, true, true, false> : k_direct_chain<float, false, true, false>))
-                           : (soa ? k_direct_chain<float, true, false, true> : k_direct_chain<float, false, false, true>);
-          C.adt_f = (float *)args[5].data_d;
-        } else {
-          C.kern = P.upd ? (P.save ? (soa ? k_direct_chain<double, true, true, true> : k_direct_chain<double, false, true, true>)
-                                   : (soa ? k_direct_chain<double, true, true, false> : k_direct_chain<double, false, true, false>))
-                         : (soa ? k_direct_chain<double, true, false, true> : k_direct_chain<double, false, false, true>);
-        }
         C.P = P;
         C.g = gg;
         C.bs = bb;
         C.chunk = chunk;
         C.q = P.q ? P.q : (double *)q;
-        C.adt = adt;
+        C.mixed = mixed;
+        C.adt = args[5].data_d;
         C.x = x;
         C.pcell = pcell;
-        if (const CompactRows *cr = compact_rows(args[0].map, st, false)) {
+        if (const CompactRows *cr = compact_rows(args[0].map)) {
           C.prow = cr->rec;
           C.pbase = cr->base;
         }
@@ -1673,9 +1744,9 @@ extern "C" void op_par_loop_airfoil_2_adt_calc(char const *name, op_set set,
       }
       flush_direct(nullptr);
     }
-    // the chains fused inside a captured step read the compact rows, built
-    // here (outside capture) at the first eager call
-    if (!ctx.capturing) (void)compact_rows(args[0].map, st, true);
+    g_last_pcell.epoch = op2h_plan_epoch();
+    g_last_pcell.map = args[0].map;
+    g_last_pcell.st = st;
     LoopTimer tm(&ctx);
     if (is_float(args[5])) {
       float *adtf = (float *)args[5].data_d;
@@ -1708,8 +1779,8 @@ extern "C" void op_par_loop_airfoil_3_res_calc(char const *name, op_set set,
   op2h_accept_deferred("chain");
   op2h_loop_begin(&ctx, 2, name, set, 8, args, OP2H_PLAN_STAGED, 256);
   hipStream_t st = (hipStream_t)ctx.stream;
-  // a fused direct chain held for this loop: launched here, before it, with
-  // or without the update's zeros in res (only an owner plan covering every
+  // a fused direct chain held for this loop: launched with it, with or
+  // without the update's zeros in res (only an owner plan covering every
   // cell can take them as known)
   bool chain = op2h_take_deferred("chain", nullptr) != 0;
   if (chain && (!op2h_fusion_enabled() || set->size == 0 || ctx.plan != OP2H_PLAN_OWNER)) {
@@ -1732,40 +1803,60 @@ extern "C" void op_par_loop_airfoil_3_res_calc(char const *name, op_set set,
       printf("op2hip: res_calc needs adt and res both FP32 (mixed mode) or both FP64\n");
       exit(-1);
     }
+    if (ctx.plan == OP2H_PLAN_OWNER) {
+      ctx.part_size = bs;
+      const op2h_owner_plan *p = op2h_plan_owner_local(&ctx);
+      PendingRes R;
+      R.A = owner_args_res(p, args, st);
+      R.lds = (mixed ? sizeof(float) : sizeof(double)) * 4 * (size_t)R.A.max_e;
+      if (R.lds > 160 * 1024) {
+        printf("op2hip: res_calc owner plan needs %zu bytes of LDS; use a smaller block\n",
+               R.lds);
+        exit(-1);
+      }
+      R.soa = soa;
+      R.mixed = mixed;
+      R.st = st;
+      R.plan = p;
+      R.epoch = op2h_plan_epoch();
+      R.x = x;
+      R.q = q;
+      R.adt = args[4].data_d;
+      R.res = args[6].data_d;
+      R.sx = sx;
+      R.sq = sq;
+      R.bs = bs;
+      R.pecell = args[6].map;
+      R.cells = args[6].dat->set;
+      // res is dead between the chain's update (which sets every cell's res
+      // to +0.0) and this loop when the plan owns every cell: the zeros are
+      // neither stored nor read
+      R.zero = chain && g_chain.P.upd && g_chain.P.mixed == mixed && g_chain.P.res == R.res &&
+               p->n_owned == R.cells->size;
+      g_last_res = R;
+      if (op2h_fusion_enabled()) {  // held for the bres_calc that follows
+        g_res = R;
+        g_res_chained = chain;
+        op2h_defer("res_owner", flush_res, nullptr);
+      } else {
+        LoopTimer tm(&ctx);
+        launch_res(tm.ext, tm.e0, tm.e1, R);
+        tm.done();
+      }
+      KCHECK(hipGetLastError());
+      account(2, set, 8, args);
+      op2h_loop_end(&ctx);
+      return;
+    }
     if (mixed) {
-      // mixed precision: atomic plan, else the owner-compute plan
+      // mixed precision: atomic plan, else the gather plan
       const float *adtf = (const float *)args[4].data_d;
       float *resf = (float *)args[6].data_d;
-      const op2h_owner_plan *owner_p = nullptr;
-      OwnerArgs OA{};
-      bool zero = false;  // as in FP64 below: res dead after the chain's update
-      if (ctx.plan == OP2H_PLAN_OWNER) {  // built before the timed region
-        ctx.part_size = bs;
-        owner_p = op2h_plan_owner_local(&ctx);
-        OA = owner_args_res(owner_p, args, st);
-        zero = chain && g_chain.P.upd && g_chain.P.mixed && g_chain.P.res_f == resf &&
-               owner_p->n_owned == args[6].dat->set->size;
-      }
-      if (chain) launch_chain(zero);
-      chain = false;
       op2h_kernel_timer_start(&ctx);
       if (ctx.plan == OP2H_PLAN_ATOMIC) {
         int g = grid_for(set->size, bs);
         if (soa) k_res_atomic_mixed<true><<<g, bs, 0, st>>>(x, q, adtf, resf, pedge, pecell, set->size, sx, sq);
         else k_res_atomic_mixed<false><<<g, bs, 0, st>>>(x, q, adtf, resf, pedge, pecell, set->size, sx, sq);
-      } else if (ctx.plan == OP2H_PLAN_OWNER) {
-        const int nblocks = owner_p->nblocks;
-        const size_t lds = sizeof(float) * 4 * (size_t)OA.max_e;
-        if (lds > 160 * 1024) {
-          printf("op2hip: res_calc owner plan needs %zu bytes of LDS; use a smaller block\n", lds);
-          exit(-1);
-        }
-        if (nblocks) {
-          auto kern = OA.csr4 ? (soa ? k_res_owner_mixed<true, true> : k_res_owner_mixed<false, true>)
-                              : (soa ? k_res_owner_mixed<true, false> : k_res_owner_mixed<false, false>);
-          launch_k(false, nullptr, nullptr, kern, nblocks, bs, lds, st, x, q, adtf, resf, OA,
-                   sx, sq, (int)zero);
-        }
       } else {
         const op2h_gather_plan *p = op2h_plan_gather(args[6].map);
         if (p->max_count > 4) {
@@ -1844,52 +1935,6 @@ extern "C" void op_par_loop_airfoil_3_res_calc(char const *name, op_set set,
         tm.done();
         break;
       }
-      case OP2H_PLAN_OWNER: {
-        ctx.part_size = bs;
-        const op2h_owner_plan *p = op2h_plan_owner_local(&ctx);
-        OwnerArgs A = owner_args_res(p, args, st);
-        const size_t lds = sizeof(double) * 4 * (size_t)A.max_e;
-        if (lds > 160 * 1024) {
-          printf("op2hip: res_calc owner plan needs %zu bytes of LDS; use a smaller block\n", lds);
-          exit(-1);
-        }
-        // res is dead between the chain's update (which sets every cell's
-        // res to +0.0) and this loop when the plan owns every cell: the
-        // zeros are neither stored nor read
-        const bool zero = chain && g_chain.P.upd && g_chain.P.res == res &&
-                          p->n_owned == args[6].dat->set->size;
-        if (chain) launch_chain(zero);
-        chain = false;
-        PendingRes R;
-        R.soa = soa;
-        R.st = st;
-        R.plan = p;
-        R.A = A;
-        R.x = x;
-        R.q = q;
-        R.adt = adt;
-        R.res = res;
-        R.sx = sx;
-        R.sq = sq;
-        R.bs = bs;
-        R.lds = lds;
-        R.pecell = args[6].map;
-        R.zero = zero;
-        g_last_res = R;
-        if (op2h_fusion_enabled()) {  // held for the bres_calc that follows
-          g_res = R;
-          op2h_defer("res_owner", flush_res, nullptr);
-          break;
-        }
-        LoopTimer tm(&ctx);
-        if (p->nblocks)
-          launch_k(tm.ext, tm.e0, tm.e1,
-                   A.csr4 ? (soa ? k_res_owner<true, true> : k_res_owner<false, true>)
-                          : (soa ? k_res_owner<true, false> : k_res_owner<false, false>),
-                   p->nblocks, bs, lds, st, x, q, adt, res, A, sx, sq, (int)zero);
-        tm.done();
-        break;
-      }
       default: {  // STAGED
         ctx.part_size = bs;
         const op2h_staged_plan *p = op2h_plan_staged(&ctx);
@@ -1930,7 +1975,6 @@ extern "C" void op_par_loop_airfoil_3_res_calc(char const *name, op_set set,
     }
     KCHECK(hipGetLastError());
   }
-  if (chain) flush_chain(nullptr);  // (every path above has launched it)
   account(2, set, 8, args);
   op2h_loop_end(&ctx);
 }
@@ -1964,21 +2008,30 @@ extern "C" void op_par_loop_airfoil_4_bres_calc(char const *name, op_set set,
     // the res_calc this loop follows, on the same dats: the two as one owner
     // launch (inside a capture), its boundary records built beforehand
     const PendingRes &L = held ? g_res : g_last_res;
-    const bool same = L.plan && L.x == x && L.q == q && L.adt == adt && L.res == res &&
-                      L.soa == soa && L.sx == sx && L.sq == sq && !is_float(args[4]) &&
+    const bool same = L.plan && L.epoch == op2h_plan_epoch() && L.x == x && L.q == q &&
+                      L.adt == args[3].data_d && L.res == args[4].data_d && L.soa == soa &&
+                      L.sx == sx && L.sq == sq && L.mixed == is_float(args[4]) &&
                       args[2].map->to == L.pecell->to && args[4].map == args[2].map;
     const BoundaryArgs *B = same ? boundary_args(L.plan, args[2].map, args[0].map, args[5].dat,
                                                  st, !ctx.capturing)
                                  : nullptr;
+    if (B && !ctx.capturing) {
+      g_last_bres.epoch = op2h_plan_epoch();
+      g_last_bres.plan = L.plan;
+      g_last_bres.rec = B->rec;
+    }
     if (held) {
       if (B) {
-        PendingRes P = g_res;
+        Half h;
+        h.chained = g_res_chained;
+        if (h.chained) h.C = g_chain;
+        h.R = g_res;
+        h.B = *B;
+        g_halves.push_back(h);
+        g_chain = PendingChain();
         g_res = PendingRes();
-        if (P.plan->nblocks)
-          launch_k(false, nullptr, nullptr, soa ? k_res_bres_owner<true> : k_res_bres_owner<false>,
-                   P.plan->nblocks, P.bs, P.lds, st, x, q, adt, res, P.A, *B, sx, sq,
-                   (int)P.zero);
-        KCHECK(hipGetLastError());
+        g_res_chained = false;
+        op2h_defer("halves", flush_halves, nullptr);  // held for the update
         account(3, set, 6, args);
         op2h_loop_end(&ctx);
         return;
@@ -2091,6 +2144,7 @@ extern "C" void op_par_loop_airfoil_5_update(char const *name, op_set set,
                                              op_arg arg6, op_arg arg7) {
   op_arg args[8] = {arg0, arg1, arg2, arg3, arg4, arg5, arg6, arg7};
   op2h_loop_ctx ctx;
+  op2h_accept_deferred("halves");
   op2h_loop_begin(&ctx, 4, name, set, 8, args, OP2H_PLAN_ATOMIC, 256);
   hipStream_t st = (hipStream_t)ctx.stream;
   int dummy;
@@ -2099,23 +2153,28 @@ extern "C" void op_par_loop_airfoil_5_update(char const *name, op_set set,
   const int bs = ctx.block_size;
   const UpdateShape shape = update_shape(set->size, bs);
   const int g = shape.g;
+  // res_calc + bres_calc recorded before this update, if any
+  const bool held = op2h_take_deferred("halves", nullptr) != 0;
+  if (held && (!op2h_fusion_enabled() || set->size == 0)) flush_halves(nullptr);
   // inside a captured graph the partials go to the runtime, whose history
   // kernel finishes both reductions of every update of the step in one pass
-  // (same tree as k_update_finish); otherwise finish them here
-  double *part_sum = nullptr, *part_max = nullptr, *slot_rms = nullptr, *slot_max = nullptr;
-  int *part_loc = nullptr, *unused = nullptr;
-  const bool deferred = op2h_gbl_partials(&ctx, 4, -1, g, &part_sum, &unused) != 0;
-  if (deferred && !op2h_gbl_partials(&ctx, 5, 7, g, &part_max, &part_loc)) {
+  // (same tree as k_update_finish); otherwise finish them here.  Where the
+  // update may run inside a half step there is room for its blocks' partials.
+  const int cap = g_halves.empty()
+                      ? g
+                      : std::max(g, std::min(g_halves.back().R.plan->nblocks, kHalfGrid));
+  double *slot_rms = nullptr, *slot_max = nullptr;
+  UpdateParts parts{};
+  const bool deferred = op2h_gbl_partials2(&ctx, 4, cap, &parts.hi, &parts.lo) != 0;
+  if (deferred && !op2h_gbl_partials(&ctx, 5, 7, cap, &parts.mx, &parts.loc)) {
     printf("op2hip: update: maxerr/errloc cannot be deferred with rms\n");
     exit(-1);
   }
   if (!deferred) {
+    if (!g_halves.empty()) flush_halves(nullptr);
     slot_rms = (double *)op2h_gbl_slot(&ctx, 4, -1);
     slot_max = (double *)op2h_gbl_slot(&ctx, 5, 7);
-    char *partials = (char *)op2h_reduct_scratch((size_t)g * 24);
-    part_sum = (double *)partials;
-    part_max = part_sum + g;
-    part_loc = (int *)(part_max + g);
+    parts = update_parts(op2h_reduct_scratch((size_t)g * kPartBytes), g);
   }
   if (is_float(args[2]) != is_float(args[3])) {
     printf("op2hip: update needs res and adt both FP32 (mixed mode) or both FP64\n");
@@ -2138,37 +2197,41 @@ extern "C" void op_par_loop_airfoil_5_update(char const *name, op_set set,
     P.chunk = shape.chunk;
     P.qold = (const double *)args[0].data_d;
     P.q = (double *)args[1].data_d;
-    if (P.mixed) {
-      P.res_f = (float *)args[2].data_d;
-      P.adt_f = (float *)args[3].data_d;
-    } else {
-      P.res = (double *)args[2].data_d;
-      P.adt = (double *)args[3].data_d;
-    }
-    P.part_sum = part_sum;
-    P.part_max = part_max;
-    P.part_loc = part_loc;
+    P.res = args[2].data_d;
+    P.adt = args[3].data_d;
+    P.cap = cap;
+    P.parts = parts;
     P.oldidx = op2h_set_old_index(set);
     op2h_defer("direct_chain", flush_direct, nullptr);
     account(4, set, 8, args);
     op2h_loop_end(&ctx);
     return;
   }
-  LoopTimer tm(&ctx);
-  if (is_float(args[2])) {
-    launch_k(tm.ext, tm.e0, nullptr, soa ? k_update_mixed<true> : k_update_mixed<false>, g, bs,
-             0, st, (const double *)args[0].data_d, (double *)args[1].data_d,
-             (float *)args[2].data_d, (const float *)args[3].data_d, set->size, s, part_sum,
-             part_max, part_loc, op2h_set_old_index(set), shape.chunk);
-  } else {
-    launch_k(tm.ext, tm.e0, nullptr, soa ? k_update<true> : k_update<false>, g, bs, 0, st,
-             (const double *)args[0].data_d, (double *)args[1].data_d,
-             (double *)args[2].data_d, (const double *)args[3].data_d, set->size, s,
-             part_sum, part_max, part_loc, op2h_set_old_index(set), shape.chunk);
+  if (deferred) {  // on its own inside a capture
+    if (!g_halves.empty()) flush_halves(nullptr);
+    op2h_gbl_partials_used(parts.hi, g);
+    op2h_gbl_partials_used(parts.mx, g);
   }
+  LoopTimer tm(&ctx);
+  PendingDirect U;
+  U.soa = soa;
+  U.st = st;
+  U.n = set->size;
+  U.s = s;
+  U.g = g;
+  U.bs = bs;
+  U.chunk = shape.chunk;
+  U.qold = (const double *)args[0].data_d;
+  U.q = (double *)args[1].data_d;
+  U.res = args[2].data_d;
+  U.adt = args[3].data_d;
+  U.parts = parts;
+  U.oldidx = op2h_set_old_index(set);
+  if (is_float(args[2])) launch_update<float>(tm.ext, tm.e0, nullptr, U);
+  else launch_update<double>(tm.ext, tm.e0, nullptr, U);
   if (!deferred)
-    launch_k(tm.ext, nullptr, tm.e1, k_update_finish, 1, kFinishThreads, 0, st, part_sum,
-             part_max, part_loc, g, slot_rms, slot_max);
+    launch_k(tm.ext, nullptr, tm.e1, k_update_finish, 1, kFinishThreads, 0, st, parts, g,
+             slot_rms, slot_max);
   tm.done();
   KCHECK(hipGetLastError());
   account(4, set, 8, args);
@@ -2186,7 +2249,7 @@ extern "C" void op_par_loop_airfoil_5_update(char const *name, op_set set,
 // ---------------------------------------------------------------------------
 namespace {
 constexpr int kNoAllocMaxParts = 2048;  // the stub's workgroup cap
-constexpr size_t kNoAllocScratchBytes = (size_t)kNoAllocMaxParts * (8 + 8 + 4);  // 40 KiB
+constexpr size_t kNoAllocScratchBytes = (size_t)kNoAllocMaxParts * kPartBytes;  // 56 KiB
 constexpr int kNoAllocMaxDevices = 64;
 void *g_scratch_addr[kNoAllocMaxDevices];  // device address of `scratch`, per device
 }  // namespace
@@ -2219,24 +2282,21 @@ extern "C" int op2h_update_noalloc(int ncell, int soa_stride, int block, const d
   }
   const UpdateShape shape = update_shape(ncell, block);  // the stub's
   const int g = shape.g;
-  if ((size_t)g * (8 + 8 + 4) > kNoAllocScratchBytes) {
+  if ((size_t)g * kPartBytes > kNoAllocScratchBytes) {
     printf("op2h_update_noalloc: %d partials exceed the %zu-byte scratch\n", g,
            kNoAllocScratchBytes);
     return -3;
   }
-  double *part_sum = (double *)g_scratch_addr[dev];
-  double *part_max = part_sum + g;
-  int *part_loc = (int *)(part_max + g);
+  const UpdateParts parts = update_parts(g_scratch_addr[dev], g);
   hipStream_t st = (hipStream_t)stream;
   // every partial the finish kernel reads is written by this call's k_update
   if (soa_stride)
-    k_update<true><<<g, block, 0, st>>>(qold, q, res, adt, ncell, soa_stride, part_sum,
-                                        part_max, part_loc, nullptr, shape.chunk);
+    k_update<double, true><<<g, block, 0, st>>>(qold, q, res, adt, ncell, soa_stride, parts,
+                                                nullptr, shape.chunk);
   else
-    k_update<false><<<g, block, 0, st>>>(qold, q, res, adt, ncell, 0, part_sum, part_max,
-                                         part_loc, nullptr, shape.chunk);
-  k_update_finish<<<1, kFinishThreads, 0, st>>>(part_sum, part_max, part_loc, g, &result->rms,
-                                               &result->maxerr);
+    k_update<double, false><<<g, block, 0, st>>>(qold, q, res, adt, ncell, 0, parts, nullptr,
+                                                 shape.chunk);
+  k_update_finish<<<1, kFinishThreads, 0, st>>>(parts, g, &result->rms, &result->maxerr);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     printf("op2h_update_noalloc: launch failed: %s\n", hipGetErrorString(e));

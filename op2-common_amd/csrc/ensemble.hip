@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(1024)
   extern __shared__ double lf[];
   for (int b = blo + xcd_block(kXcds); b < bhi; b += gridDim.x) {
     const unsigned long long t0 = stamp_now(S);
-    owner_res_block<false, true>(b, x, q, adt, res, P, 0, 0, lf, zero != 0);
+    owner_res_block<double, false, true>(b, x, q, adt, res, P, 0, 0, lf, zero != 0);
     __syncthreads();  // the next patch rewrites lf
     if (S.t && threadIdx.x == 0) stamp(S, b, t0);
   }
@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(1024)
   extern __shared__ double lf[];
   for (int b = blo + xcd_block(kXcds); b < bhi; b += gridDim.x) {
     const unsigned long long t0 = stamp_now(S);
-    owner_res_bres_block<false, true>(b, x, q, adt, res, P, B, 0, 0, lf, zero != 0);
+    owner_res_bres_block<double, false, true>(b, x, q, adt, res, P, B, 0, 0, lf, zero != 0);
     __syncthreads();  // the next patch rewrites lf
     if (S.t && threadIdx.x == 0) stamp(S, b, t0);
   }

@@ -148,11 +148,13 @@ struct Runtime {
   hipGraphExec_t graph_exec = nullptr;
   std::vector<DeferredGbl> deferred;
   std::vector<std::pair<void *, size_t>> history_sources;  // device slots
-  // deferred reductions: slot -> (kind 1 sum / 2 max / 3 min, nparts, vals, locs)
+  // deferred reductions: slot -> (kind 1 sum / 2 max / 3 min / 4 sum of
+  // pairs, nparts, vals, locs, lows)
   struct Partials {
     int kind, nparts;
     const double *vals;
     const int *locs;
+    const double *lows;
   };
   std::map<void *, Partials> partial_of_slot;
   char *partial_pool = nullptr;
@@ -2015,22 +2017,24 @@ extern "C" void *op2h_gbl_slot(op2h_loop_ctx *ctx, int argi, int info_argi) {
   return slot.first;
 }
 
-extern "C" int op2h_gbl_partials(op2h_loop_ctx *ctx, int argi, int info_argi,
-                                 int nparts, double **vals, int **locs) {
+namespace {
+// The pool's next `nparts` partials for gbl arg `argi`, registered for the
+// history kernel; `pairs`: the sum's hi and lo parts.
+int take_partials(op2h_loop_ctx *ctx, int argi, int info_argi, int nparts, bool pairs,
+                  double **vals, int **locs, double **lows) {
   Runtime &R = rt();
-  *vals = nullptr;
-  *locs = nullptr;
   const op_arg &a = ctx->args[argi];
   if (!R.capturing || !R.partial_pool || nparts < 1 ||
       nparts > op2h_red::kRedThreads * op2h_red::kRedMaxLoads || a.dim != 1 ||
       type_code(a.type) != 0)
     return 0;
   const bool extremum = a.acc == OP_MIN || a.acc == OP_MAX;
-  if (a.acc != OP_INC && !extremum) return 0;
+  if (a.acc != OP_INC && (!extremum || pairs)) return 0;
   if (extremum && info_argi >= 0 &&
       (ctx->args[info_argi].dim != 1 || type_code(ctx->args[info_argi].type) != 2))
     return 0;
-  const size_t need = (size_t)nparts * (sizeof(double) + (extremum ? sizeof(int) : 0));
+  const size_t need = (size_t)nparts * (sizeof(double) * (pairs ? 2 : 1) +
+                                        (extremum ? sizeof(int) : 0));
   const size_t at = (R.partial_pool_next + 255) / 256 * 256;
   if (at + need > R.partial_pool_bytes) {
     printf("op2hip: deferred reductions of one graph exceed %zu bytes\n",
@@ -2039,16 +2043,38 @@ extern "C" int op2h_gbl_partials(op2h_loop_ctx *ctx, int argi, int info_argi,
   }
   R.partial_pool_next = at + need;
   void *slot = op2h_gbl_slot(ctx, argi, info_argi);
+  char *tail = R.partial_pool + at + (size_t)nparts * sizeof(double);
   Runtime::Partials P;
-  P.kind = a.acc == OP_INC ? 1 : a.acc == OP_MAX ? 2 : 3;
+  P.kind = pairs ? 4 : a.acc == OP_INC ? 1 : a.acc == OP_MAX ? 2 : 3;
   P.nparts = nparts;
   P.vals = (const double *)(R.partial_pool + at);
-  P.locs = extremum ? (const int *)(R.partial_pool + at + (size_t)nparts * sizeof(double))
-                    : nullptr;
+  P.locs = extremum ? (const int *)tail : nullptr;
+  P.lows = pairs ? (const double *)tail : nullptr;
   R.partial_of_slot[slot] = P;
   *vals = (double *)P.vals;
-  *locs = (int *)P.locs;
+  if (locs) *locs = (int *)P.locs;
+  if (lows) *lows = (double *)P.lows;
   return 1;
+}
+}  // namespace
+
+extern "C" int op2h_gbl_partials(op2h_loop_ctx *ctx, int argi, int info_argi,
+                                 int nparts, double **vals, int **locs) {
+  *vals = nullptr;
+  *locs = nullptr;
+  return take_partials(ctx, argi, info_argi, nparts, false, vals, locs, nullptr);
+}
+
+extern "C" int op2h_gbl_partials2(op2h_loop_ctx *ctx, int argi, int nparts, double **hi,
+                                  double **lo) {
+  *hi = nullptr;
+  *lo = nullptr;
+  return take_partials(ctx, argi, -1, nparts, true, hi, nullptr, lo);
+}
+
+extern "C" void op2h_gbl_partials_used(const double *vals, int nparts) {
+  for (auto &kv : rt().partial_of_slot)
+    if (kv.second.vals == vals) kv.second.nparts = std::min(kv.second.nparts, nparts);
 }
 
 extern "C" void *op2h_reduct_scratch(size_t bytes) {
@@ -2304,6 +2330,11 @@ extern "C" int op2h_color_plan_download(const op2h_color_plan *p,
 // graph capture
 // ===========================================================================
 namespace {
+std::vector<op2h_capture_hook> &capture_hooks() {
+  static std::vector<op2h_capture_hook> hooks;
+  return hooks;
+}
+
 constexpr int kSlotPool = 128;
 constexpr int kHistSources = 64;
 constexpr size_t kHistoryBytes = 64u << 20;
@@ -2311,9 +2342,10 @@ constexpr size_t kHistoryBytes = 64u << 20;
 struct HistSources {
   const unsigned long long *p[kHistSources];  // slot words, or partial values
   const int *locs[kHistSources];              // partial payloads (max/min)
+  const double *lows[kHistSources];           // low parts (sums of pairs)
   int words[kHistSources];
   int off[kHistSources];     // first word of the source in a record
-  int kind[kHistSources];    // 0 copy the slot, 1 sum, 2 max, 3 min of partials
+  int kind[kHistSources];    // 0 copy the slot, 1 sum, 2 max, 3 min, 4 sum of pairs
   int nparts[kHistSources];
   int n;
   int red[kHistSources];     // indices of the deferred reductions
@@ -2332,7 +2364,7 @@ struct HistSources {
 __global__ void __launch_bounds__(op2h_red::kRedThreads)
     history_append(HistSources src, double *hist, unsigned long long *count,
                    unsigned int *done, int capacity, int total_words) {
-  __shared__ double s_v[op2h_red::kRedThreads / 64];
+  __shared__ double s_v[op2h_red::kRedThreads / 64], s_lo[op2h_red::kRedThreads / 64];
   __shared__ int s_l[op2h_red::kRedThreads / 64];
   const unsigned long long c = *count;
   const size_t base = (size_t)(c % (unsigned long long)capacity) * total_words;
@@ -2345,8 +2377,8 @@ __global__ void __launch_bounds__(op2h_red::kRedThreads)
   if (b < src.nred) {
     const int s = src.red[b];
     const op2h_red::ValLoc v = op2h_red::group_reduce(
-        reinterpret_cast<const double *>(src.p[s]), src.locs[s], src.nparts[s], src.kind[s], t,
-        s_v, s_l);
+        reinterpret_cast<const double *>(src.p[s]), src.locs[s], src.lows[s], src.nparts[s],
+        src.kind[s], t, s_v, s_l, s_lo);
     if (t == 0) {
       hist[base + src.off[s]] = v.v;
       if (src.words[s] > 1)  // the info int in the low half of the next word
@@ -2364,6 +2396,10 @@ __global__ void __launch_bounds__(op2h_red::kRedThreads)
 }
 }  // namespace
 
+extern "C" void op2h_register_capture_hook(op2h_capture_hook hook) {
+  capture_hooks().push_back(hook);
+}
+
 extern "C" int op2h_graph_begin(void) {
   Runtime &R = rt();
   ensure_init();
@@ -2374,6 +2410,7 @@ extern "C" int op2h_graph_begin(void) {
   HIPCHECK(hipStreamSynchronize(R.stream));
   R.deferred.clear();
   R.history_sources.clear();
+  for (op2h_capture_hook h : capture_hooks()) h();
   // everything a capture needs is allocated before capture starts
   for (int i = 0; i < kSlotPool; ++i) {
     std::pair<void *, void *> slot;
@@ -2419,6 +2456,7 @@ extern "C" int op2h_graph_end(void) {
     if (pi != R.partial_of_slot.end()) {
       src.p[src.n] = (const unsigned long long *)pi->second.vals;
       src.locs[src.n] = pi->second.locs;
+      src.lows[src.n] = pi->second.lows;
       src.kind[src.n] = pi->second.kind;
       src.nparts[src.n] = pi->second.nparts;
       src.red[src.nred++] = src.n;

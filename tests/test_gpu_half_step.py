@@ -1,0 +1,158 @@
+"""Captured airfoil steps as fused half steps (one launch per half step over
+the owner plan's patches): bit for bit the unfused loops, at the edges of the
+patches (fewer cells than one, partly filled last ones, more staged cells or
+nodes than two per thread), on every ordering, layout and precision, where the
+patches do not fit their 16-bit lists and the loops run unfused, and for
+captured sequences that are not whole time steps."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import op2amd
+import op2amd.api as api
+from oracle import oracle
+from test_gpu_loops import App, inputs
+
+pytestmark = pytest.mark.gpu
+KEYS = ("rms", "rms_k0", "maxerr", "errloc", "q")
+
+
+def fused_and_not(mesh, niter, **kw):
+    kw = dict(dict(mode="graphed", plan_res="owner", plan_bres="gather", graph_steps=4), **kw)
+    fused = op2amd.airfoil.run(mesh, niter, **kw)
+    api.op2h_set_fusion(0)
+    try:
+        return fused, op2amd.airfoil.run(mesh, niter, **kw)
+    finally:
+        api.op2h_set_fusion(1)
+
+
+@pytest.mark.parametrize("I,J,ordering,block", [
+    (2, 2, "structured", 64), (9, 7, "structured", 64), (16, 8, "random", 128),
+    (33, 31, "rcm", 64), (61, 47, "random", 192), (90, 90, "hilbert", 256),
+    (100, 83, "structured", 1024), (64, 64, "rcm", 512)])
+@pytest.mark.parametrize("kw", [dict(), dict(soa=True), dict(mixed=True)],
+                         ids=["fp64", "soa", "mixed"])
+def test_half_steps_equal_unfused_loops(I, J, ordering, block, kw):
+    mesh = op2amd.mesh.generate(I, J, 3, ordering)
+    fused, plain = fused_and_not(mesh, 29, block_res=block, **kw)
+    for k in KEYS:
+        assert np.array_equal(fused[k], plain[k]), k
+    if not kw:
+        ref = oracle.airfoil_run(mesh, 29, 1, "seq")
+        assert np.array_equal(fused["q"], ref["q"])
+
+
+@pytest.mark.parametrize("renumber", [False, "transparent"])
+def test_wide_patches_run_unfused(renumber):
+    """75,000 randomly numbered cells: a patch's cells span more than 16 bits
+    unless the device renumbers them."""
+    mesh = op2amd.mesh.generate(300, 250, 5, "random")
+    fused, plain = fused_and_not(mesh, 13, block_res=128, renumber=renumber)
+    for k in KEYS:
+        assert np.array_equal(fused[k], plain[k]), k
+
+
+STEP = ["save_soln"] + 2 * ["adt_calc", "res_calc", "bres_calc", "update"]
+SEQUENCES = {
+    "step": STEP,
+    "three steps": 3 * STEP,
+    "step, then one stage": STEP + ["save_soln", "adt_calc", "res_calc", "bres_calc", "update"],
+    "one stage, twice": 2 * ["save_soln", "adt_calc", "res_calc", "bres_calc", "update"],
+    "ends on save_soln": STEP + ["save_soln"],
+    "ends on adt_calc": 2 * STEP + ["save_soln", "adt_calc"],
+    "ends on res_calc": STEP + ["save_soln", "adt_calc", "res_calc"],
+    "ends on bres_calc": STEP + STEP[:-1],
+    "starts inside a step": STEP[1:] + STEP,
+    "no save_soln": STEP[1:] + STEP[1:],
+    "a second adt_calc": STEP[:2] + ["adt_calc"] + STEP[2:] + STEP,
+}
+
+
+class Program(App):
+    def save_soln(self):
+        api.loops["op_par_loop_airfoil_1_save_soln"](
+            b"save_soln", self.cells, self.d(self.q, -1, None, 4, "double", api.OP_READ),
+            self.d(self.qold, -1, None, 4, "double", api.OP_WRITE))
+
+    def play(self, names):
+        g = (C.c_double(0.0), C.c_double(0.0), C.c_int(0))
+        for n in names:
+            getattr(self, n)(*(g if n == "update" else ()))
+
+    def state(self):
+        n = self.m.ncell
+        for d in (self.q, self.qold, self.adt, self.res):
+            api.lib.op_download_dat(d)  # (a replayed graph marks no dat as newer on the device)
+        return [self.fetch(d, s) for d, s in ((self.q, (n, 4)), (self.qold, (n, 4)),
+                                              (self.adt, (n,)), (self.res, (n, 4)))]
+
+
+@pytest.mark.parametrize("soa", [False, True], ids=["aos", "soa"])
+@pytest.mark.parametrize("name", SEQUENCES)
+def test_captured_sequences_leave_every_dat_as_eager_loops_do(name, soa):
+    """Three replays of a captured sequence, each followed by a fetch of q,
+    qold, adt and res, against the same loops run eagerly."""
+    mesh = op2amd.mesh.generate(70, 41, 2, "rcm")
+    q, res = inputs(mesh, 4)
+
+    def run(captured):
+        app = Program(mesh, q, res, soa=soa)
+        try:
+            api.op2h_set_sync_mode(api.SYNC_GBL_ONLY)
+            api.op2h_set_loop_plan(b"res_calc", api.PLAN_OWNER, 128)
+            api.op2h_set_loop_plan(b"bres_calc", api.PLAN_GATHER, 128)
+            app.play(STEP)  # builds the plans
+            out = []
+            if captured:
+                assert api.lib.op2h_graph_begin() == 0
+                app.play(SEQUENCES[name])
+                assert api.lib.op2h_graph_end() == 0
+            for _ in range(3):
+                if captured:
+                    assert api.lib.op2h_graph_launch(1) == 0
+                    api.op2h_device_sync()
+                else:
+                    app.play(SEQUENCES[name])
+                out.append(app.state())
+            return out
+        finally:
+            app.close()
+
+    for eager, graph in zip(run(False), run(True)):
+        for a, b in zip(eager, graph):
+            assert np.array_equal(a, b)
+
+
+def test_update_reductions_do_not_depend_on_the_grouping():
+    """rms is a sum of unevaluated pairs rounded once: the same bits for every
+    workgroup size and launch shape, within 2^-52 of the exactly rounded sum
+    (each cell's own four squares are summed in double first: 3 roundings of
+    positive terms, 1.5 * 2^-52), also with infinities and NaN."""
+    import math
+    from test_zz_no_alloc import inputs as arrays, stub_update
+    n = 70_001
+    qold, q, res, adt = arrays(n, 9)
+    got = set()
+    for block in (64, 256, 1024):
+        api.init()
+        try:
+            api.op2h_set_loop_plan(b"update", 0, block)
+        finally:
+            api.op_exit()
+        for mode in (0, 1):
+            api.op2h_set_streaming(mode)
+            try:
+                got.add(stub_update(qold, q, res, adt, False)[2])
+            finally:
+                api.op2h_set_streaming(-1)
+    assert len(got) == 1
+    exact = math.fsum(((res / adt[:, None]) ** 2).ravel())
+    # adti * res rounds twice where res / adt rounds once: another 2 * 2^-53 per
+    # square, doubled by squaring
+    assert abs(got.pop() - exact) <= 5 * 2.0 ** -52 * exact
+    res[123, 2] = np.inf
+    assert stub_update(qold, q, res, adt, False)[2] == np.inf
+    res[60_000, 1] = np.nan
+    assert np.isnan(stub_update(qold, q, res, adt, False)[2])
