@@ -143,3 +143,29 @@ def test_runtime_picks_each_loop_plan_with_the_model():
     assert pred[cands.index(chosen)] <= pred.min() + 1e-4
     assert r["chosen"]["save_soln"][1] in cm.BLOCKS
     assert pointwise_rel_err(r["rms"], g["rms"][:200]) <= 1e-10
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nin,hidden", [(1, 64), (4, 64), (21, 64), (63, 64), (64, 64), (65, 64),
+                                        (22, 48)])
+def test_row_kernels_at_the_edges_of_their_tiles(nin, hidden):
+    """Networks of 64 hidden units and at most 64 inputs go through the row
+    kernels (16 samples a wave, 32 a workgroup, 256 a gradient split; forward
+    passes of up to 65536 input values through pinned host memory), others
+    through the general products: forward pass and gradients of both against
+    the float64 oracle on either side of each edge, within 1e-4 of the
+    largest value: FP32 sums of at most 65536 terms in splits of 256 (at most
+    256 roundings within a split and 256 over the splits, 512 * 2^-24 = 3e-5
+    if they all went one way)."""
+    m = op2amd.costmodel.MLP(nin, hidden, seed=5)
+    p = m.params()
+    rng = np.random.default_rng(nin)
+    for n in sorted({1, 15, 16, 17, 32, 33, 256, 257, 65536 // nin, 65536 // nin + 1}):
+        x = rng.standard_normal((n, nin)).astype(np.float32)
+        t = rng.standard_normal(n).astype(np.float32)
+        y, _ = mlp_ref.forward(p, x.astype(np.float64), nin, hidden)
+        assert np.max(np.abs(m.forward(x) - y)) <= 1e-4 * max(1.0, np.max(np.abs(y))), n
+        loss, grad = m.loss_grad(x, t)
+        rl, rg = mlp_ref.loss_grad(p, x, t, nin, hidden)
+        assert abs(loss - rl) <= 1e-4 * rl, n
+        assert np.max(np.abs(grad - rg)) <= 1e-4 * np.max(np.abs(rg)), n
