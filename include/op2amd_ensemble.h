@@ -71,7 +71,8 @@ typedef struct {
                         adt_calc launches and of bres_calc picked by timing
                         the first ten steps (candidates 64..1024, one per
                         step, each twice; a candidate's time is its faster
-                        step; the results do not depend on them) */
+                        step; the results do not depend on them); half steps
+                        have nothing to tune */
   int max_workgroups; /* > 0: at most this many workgroups per launch (each
                          then walks more work items); 0: as many as the GPU
                          holds at once */

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "airfoil_device.h"
+#include "airfoil_patch.h"
 #include "op2h_plan_build.h"
 
 #define ECHECK(x)                                                            \
@@ -40,6 +41,7 @@ using namespace op2_dev;
 constexpr int kTile = 1024;          // cells per tile of the update chain
 constexpr int kGroups = kTile / 64;  // reduction groups (one wave's cells) per tile
 constexpr int kPatch = 256;          // default cells per owner patch of res_calc
+constexpr int kGraphSteps = 10;      // time steps per captured graph
 
 struct SplitMix64 {
   uint64_t s;
@@ -158,36 +160,38 @@ __global__ void k_ens_bres(const double *__restrict x, const double *__restrict 
   }
 }
 
-struct MaxLoc {
-  double v;
-  int loc;
-};
+using op2h_red::MaxLoc;
+using op2h_red::Sum2;
+using op2h_red::UpdateAcc;
+using op2h_red::UpdateParts;
 
-__device__ __forceinline__ MaxLoc maxloc_combine(MaxLoc a, MaxLoc b) {
-  if (b.v > a.v || (b.v == a.v && b.loc < a.loc)) return b;
-  return a;
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-__device__ __forceinline__ MaxLoc wave_maxloc(MaxLoc m) {
-  for (int o = 32; o > 0; o >>= 1) {
-    MaxLoc t;
-    t.v = __shfl_xor(m.v, o, 64);
-    t.loc = __shfl_xor(m.loc, o, 64);
-    m = maxloc_combine(m, t);
+// A half time step of every member in one pass (half_step_patch), persistent
+// over the owner patches [plo, phi): res_calc, bres_calc with the member's own
+// free stream, update and the adt_calc that follows, q and adt written to
+// their other copies.  RED: the update's partial of each patch (one member's
+// cells) at its index.  member: patch -> {member, its first cell}.  1.1 million
+// cells in 16 members: 81 us a step, 147 as chains and res_calc + bres_calc
+// launches of one step per graph; 64 members of up to 160x80: 45 against 66.
+template <bool RED>
+__global__ void __launch_bounds__(1024)
+    k_ens_half(HalfArgs<double> H, PatchArgs P, BoundaryArgs B, const int2 *__restrict member,
+               int nc, int nn, int plo, int phi, UpdateParts parts, Stamps S) {
+  extern __shared__ double lf[];
+  for (int b = plo + xcd_block(kXcds); b < phi; b += gridDim.x) {
+    const unsigned long long t0 = stamp_now(S);
+    UpdateAcc acc;
+    half_step_patch<double, false, true>(b, H, P, B, member[b].y, lf, nc, nn, acc);
+    if (RED) op2h_red::write_partial(acc, parts, b);
+    __syncthreads();  // the next patch restages the LDS
+    if (S.t && threadIdx.x == 0) stamp(S, b, t0);
   }
-  return m;
 }
 
 // update, save_soln and adt_calc of each cell in one pass, persistent over
 // tiles [tlo, thi) of <= kTile cells of one member ({first cell, member}):
 //  UPD   q = update(qold, res, adt) (update.h), the member's rms/maxerr/errloc
-//        partials when RED: one per 64-cell group (a wave's sum), at
-//        part_*[tile * kGroups + group];
+//        partials when RED: one per 64-cell group (a wave's share), at
+//        index tile * kGroups + group;
 //  SAVE  qold = q (save_soln.h), the next time step's;
 //  then  adt = adt_calc(x, q) (adt_calc.h) for the next half step.
 // DEAD: the update's zeros in res are not stored (res_calc, which comes next,
@@ -203,8 +207,7 @@ __global__ void __launch_bounds__(kTile)
                 double *__restrict res, double *adt, const int4 *__restrict pcell,
                 const uint2 *__restrict prow, const int *__restrict pbase,
                 const int2 *__restrict tiles, const int *__restrict coff, int tlo, int thi,
-                double *__restrict part_sum, double *__restrict part_max,
-                int *__restrict part_loc, Stamps S) {
+                UpdateParts parts, Stamps S) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int t = tlo + xcd_block(kXcds); t < thi; t += gridDim.x) {
     const unsigned long long t0 = stamp_now(S);
@@ -212,18 +215,15 @@ __global__ void __launch_bounds__(kTile)
     const int base = coff[tl.y], end = min(tl.x + kTile, coff[tl.y + 1]);
     for (int r = 0; r < kTile; r += blockDim.x) {
       const int c = tl.x + r + (int)threadIdx.x;
-      double rms = 0.0;
-      MaxLoc ml{-INFINITY, 0x7fffffff};
+      UpdateAcc acc;
       if (c < end) {
         double qn[4];
         if (UPD) {
-          double qo[4], rr[4], a = adt[c], mx = ml.v;
-          int loc = ml.loc, local = c - base;  // index within the member
+          double qo[4], rr[4], a = adt[c];
+          int local = c - base;  // index within the member
           ld4<false>(qold, c, 0, qo);
           ld4<false>(res, c, 0, rr);
-          op2_k::update(qo, qn, rr, &a, &rms, &mx, &local, &loc);
-          ml.v = mx;
-          ml.loc = loc;
+          op2_k::update(qo, qn, rr, &a, &acc.rms.hi, &acc.ml.v, &local, &acc.ml.loc);
           st4<false>(q, c, 0, qn);
           if (!DEAD) st4<false>(res, c, 0, rr);
         } else {
@@ -248,13 +248,13 @@ __global__ void __launch_bounds__(kTile)
         adt[c] = a2;
       }
       if (RED) {
-        rms = wave_sum(rms);
-        ml = wave_maxloc(ml);
+        op2h_red::wave_join(acc);
         if (lane == 0) {
           const size_t g = (size_t)t * kGroups + (r >> 6) + wave;
-          part_sum[g] = rms;
-          part_max[g] = ml.v;
-          part_loc[g] = ml.loc;
+          parts.hi[g] = acc.rms.hi;
+          parts.lo[g] = acc.rms.lo;
+          parts.mx[g] = acc.ml.v;
+          parts.loc[g] = acc.ml.loc;
         }
       }
     }
@@ -267,63 +267,53 @@ __global__ void __launch_bounds__(kTile)
   }
 }
 
-// One workgroup per member: its tiles' partials, each summed over its groups
-// in order, then over the tiles.
+// One workgroup per member of [mlo, mlo + gridDim.x): its partials
+// [off[m] per, off[m + 1] per), thread t's every 256th of them, then the
+// waves; the member's results go to the step's history record.  The step is
+// complete, and the record count advanced, when `members` workgroups have done
+// so (one launch, or one per member): the last to take a ticket on `done`,
+// after a release fence that orders its writes and stamps before it, advances
+// the count and resets the ticket.  (A launch of its own for the record cost
+// 4 us a step.)
 __global__ void __launch_bounds__(256)
-    k_ens_finish(const double *__restrict part_sum, const double *__restrict part_max,
-                 const int *__restrict part_loc, const int *__restrict mesh_tile_off,
-                 int mlo, double *__restrict slots, Stamps S) {
-  __shared__ double s_sum[4];
-  __shared__ double s_max[4];
+    k_ens_finish(UpdateParts parts, const int *__restrict off, int per, int mlo, int members,
+                 double *__restrict hist, unsigned long long *count, unsigned int *done,
+                 int capacity, Stamps S) {
+  __shared__ double s_hi[4], s_lo[4], s_max[4];
   __shared__ int s_loc[4];
   const int m = mlo + blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const unsigned long long t0 = stamp_now(S);
-  double tot = 0.0;
-  MaxLoc tm{-INFINITY, 0x7fffffff};
-  for (int t = mesh_tile_off[m] + tid; t < mesh_tile_off[m + 1]; t += 256) {
-    // the tile's partial: its groups in order
-    double ts = 0.0;
-    MaxLoc tg{-INFINITY, 0x7fffffff};
-    for (int g = 0; g < kGroups; ++g) {
-      const size_t k = (size_t)t * kGroups + g;
-      ts += part_sum[k];
-      tg = maxloc_combine(tg, MaxLoc{part_max[k], part_loc[k]});
-    }
-    tot += ts;
-    tm = maxloc_combine(tm, tg);
+  const unsigned long long t0 = stamp_now(S), c = *count;
+  double *slots = hist + (size_t)(c % (unsigned long long)capacity) * 3 * members;
+  UpdateAcc a;
+  for (int k = off[m] * per + tid; k < off[m + 1] * per; k += 256) {
+    a.rms = op2h_red::sum2_join(a.rms, Sum2{parts.hi[k], parts.lo[k]});
+    a.ml = op2h_red::maxloc_combine(a.ml, MaxLoc{parts.mx[k], parts.loc[k]});
   }
-  tot = wave_sum(tot);
-  tm = wave_maxloc(tm);
+  op2h_red::wave_join(a);
   if (lane == 0) {
-    s_sum[wave] = tot;
-    s_max[wave] = tm.v;
-    s_loc[wave] = tm.loc;
+    s_hi[wave] = a.rms.hi;
+    s_lo[wave] = a.rms.lo;
+    s_max[wave] = a.ml.v;
+    s_loc[wave] = a.ml.loc;
   }
   __syncthreads();
   if (tid == 0) {
-    double t = 0.0;
-    MaxLoc mm{-INFINITY, 0x7fffffff};
+    UpdateAcc r;
     for (int w = 0; w < 4; ++w) {
-      t += s_sum[w];
-      mm = maxloc_combine(mm, MaxLoc{s_max[w], s_loc[w]});
+      r.rms = op2h_red::sum2_join(r.rms, Sum2{s_hi[w], s_lo[w]});
+      r.ml = op2h_red::maxloc_combine(r.ml, MaxLoc{s_max[w], s_loc[w]});
     }
-    slots[3 * (size_t)m] = t;
-    slots[3 * (size_t)m + 1] = mm.v;
-    slots[3 * (size_t)m + 2] = (double)mm.loc;
+    slots[3 * (size_t)m] = op2h_red::sum2_value(r.rms);
+    slots[3 * (size_t)m + 1] = r.ml.v;
+    slots[3 * (size_t)m + 2] = (double)r.ml.loc;
     if (S.t) stamp(S, m, t0);
+    __threadfence();
+    if (atomicAdd(done, 1u) == (unsigned)members - 1) {
+      *done = 0u;
+      *count = c + 1;
+    }
   }
-}
-
-// history[record][k] = slots[k]; one workgroup; the counter advances once.
-__global__ void k_ens_history(const double *__restrict slots, int nwords,
-                              double *__restrict hist, unsigned long long *count,
-                              int capacity) {
-  unsigned long long c = *count;
-  size_t base = (size_t)(c % (unsigned long long)capacity) * nwords;
-  for (int k = threadIdx.x; k < nwords; k += blockDim.x) hist[base + k] = slots[k];
-  __syncthreads();
-  if (threadIdx.x == 0) *count = c + 1;
 }
 
 // ---- host -----------------------------------------------------------------
@@ -631,20 +621,45 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
   int2 *d_tiles = dev_upload(tiles, keep);
   int *d_coff = dev_upload(coff, keep);
   int *d_mtoff = dev_upload(mesh_tile_off, keep);
-  double *d_psum = dev_alloc<double>((size_t)ntiles * kGroups, keep);
-  double *d_pmax = dev_alloc<double>((size_t)ntiles * kGroups, keep);
-  int *d_ploc = dev_alloc<int>((size_t)ntiles * kGroups, keep);
-  double *d_slots = dev_alloc<double>(3 * (size_t)M, keep);
+  // the half steps' memory: where bres_calc is not kept apart and every patch
+  // fits its lists, each half step is one launch (k_ens_half); else the chains
+  // and res_calc + bres_calc
+  hipStream_t st;
+  ECHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+  PatchArgs PA{};
+  int pa_nc = 0, pa_nn = 0;
+  bool half = fused && npatch > 0 &&
+              build_patches(OA, npatch, BA.rec, d_cell, Nc, st,
+                            [&](size_t bytes) { return dev_alloc<char>(bytes, keep); }, &PA,
+                            &pa_nc, &pa_nn);
+  const size_t half_lds = patch_lds_bytes<double>(pa_nc, pa_nn);
+  half = half && half_lds <= 64 * 1024;
+  double *d_q2 = half ? dev_alloc<double>(4 * (size_t)Nc, keep) : nullptr;
+  double *d_adt2 = half ? dev_alloc<double>(Nc, keep) : nullptr;
+  std::vector<int2> pmember(npatch);
+  for (int m = 0; m < M; ++m)
+    for (int b = mblk[m]; b < mblk[m + 1]; ++b) pmember[b] = make_int2(m, coff[m]);
+  const int2 *d_pmember = half ? dev_upload(pmember, keep) : nullptr;
+  const int *d_mblk = half ? dev_upload(mblk, keep) : nullptr;
+  const size_t nparts = half ? npatch : (size_t)ntiles * kGroups;
+  UpdateParts parts;
+  parts.hi = dev_alloc<double>(3 * nparts, keep);
+  parts.lo = parts.hi + nparts;
+  parts.mx = parts.lo + nparts;
+  parts.loc = dev_alloc<int>(nparts, keep);
   const int hist_words = 3 * M;
   const int capacity = o->niter;
   double *d_hist = dev_alloc<double>((size_t)hist_words * capacity, keep);
   unsigned long long *d_count = dev_alloc<unsigned long long>(1, keep);
+  unsigned int *d_done = dev_alloc<unsigned int>(1, keep);
   // per-step stamp layout, in launch order: res_calc, bres_calc, the chain,
   // twice, then the per-member finish
-  const int off_res[2] = {0, npatch + nbitem + ntiles};
-  const int off_bres[2] = {npatch, 2 * npatch + nbitem + ntiles};
-  const int off_chain[2] = {npatch + nbitem, 2 * (npatch + nbitem) + ntiles};
-  const int off_fin = 2 * (npatch + nbitem + ntiles), per_step = off_fin + M;
+  // (half steps: the patches, twice)
+  const int nchain = half ? 0 : ntiles;
+  const int off_res[2] = {0, npatch + nbitem + nchain};
+  const int off_bres[2] = {npatch, 2 * npatch + nbitem + nchain};
+  const int off_chain[2] = {npatch + nbitem, 2 * (npatch + nbitem) + nchain};
+  const int off_fin = 2 * (npatch + nbitem + nchain), per_step = off_fin + M;
   const bool stamps = o->batched && o->member_timing;
   unsigned long long *d_stamp =
       stamps ? dev_alloc<unsigned long long>(2 * (size_t)per_step * capacity, keep) : nullptr;
@@ -656,15 +671,13 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
     ECHECK(hipMemcpyToSymbol(HIP_SYMBOL(cfl_d), &cfl, sizeof(double)));
     ECHECK(hipMemcpyToSymbol(HIP_SYMBOL(eps_d), &eps, sizeof(double)));
   }
-  hipStream_t st;
-  ECHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
   ECHECK(hipDeviceSynchronize());
 
   int nsm = 0;
   ECHECK(hipDeviceGetAttribute(&nsm, hipDeviceAttributeMultiprocessorCount, 0));
   using ChainFn = void (*)(const double *, double *, double *, double *, double *,
                            const int4 *, const uint2 *, const int *, const int2 *, const int *,
-                           int, int, double *, double *, int *, Stamps);
+                           int, int, UpdateParts, Stamps);
   const ChainFn k_prologue = k_ens_chain<false, true, false, false>;
   const ChainFn k_chain0 = dead ? k_ens_chain<true, false, false, true>
                                 : k_ens_chain<true, false, false, false>;
@@ -694,6 +707,11 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
                       blk[1], res_lds);
     cap[2] = resident((const void *)k_ens_bres, blk[2], 0) * (blk[2] / 64);  // waves
     cap[3] = resident((const void *)k_chain1, blk[3], 0);
+    if (half) {  // one launch per half step over the patches
+      blk[0] = blk[3] = patch;
+      cap[0] = resident((const void *)k_ens_half<false>, patch, half_lds);
+      cap[1] = cap[3] = resident((const void *)k_ens_half<true>, patch, half_lds);
+    }
   };
   set_caps();
   const int res_zero = dead ? 1 : 0;
@@ -707,7 +725,7 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
     if (t1 > t0)
       k_prologue<<<std::min(t1 - t0, cap[0]), blk[0], 0, st>>>(
           d_x, d_qold, d_q, d_res, d_adt, d_cell, d_crow, d_cbase, d_tiles, d_coff, t0, t1,
-          d_psum, d_pmax, d_ploc, Stamps{nullptr, d_count, per_step, capacity, 0});
+          parts, Stamps{nullptr, d_count, per_step, capacity, 0});
   };
   // one time step of members [mlo, mhi): twice res_calc and bres_calc (one
   // launch when fused) and the chain, then the per-member reductions; with
@@ -722,7 +740,25 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
     auto mark = [&]() {
       if (ev) ECHECK(hipEventRecord(ev[e++], st));
     };
-    for (int k = 0; k < 2; ++k) {
+    // half steps: q, adt to their other copies and back, the second update
+    // reading the step's first q from the array it overwrites
+    for (int k = 0; k < 2 && half; ++k) {
+      HalfArgs<double> H{};
+      H.x = d_x;
+      H.q = k ? d_q2 : d_q;
+      H.adt = k ? d_adt2 : d_adt;
+      H.qold = k ? d_q : nullptr;
+      H.q_out = k ? d_q : d_q2;
+      H.adt_out = k ? d_adt : d_adt2;
+      H.flags = kHalfAdt;
+      // every workgroup walks the same number of patches, give or take one
+      const int most = std::max(1, std::min(p1 - p0, cap[3 * k]));
+      const int rounds = (p1 - p0 + most - 1) / most, grid = (p1 - p0 + rounds - 1) / std::max(1, rounds);
+      if (p1 > p0)
+        (k ? k_ens_half<true> : k_ens_half<false>)<<<grid, patch, half_lds, st>>>(
+            H, PA, BA, d_pmember, pa_nc, pa_nn, p0, p1, parts, S_at(off_res[k]));
+    }
+    for (int k = 0; k < 2 && !half; ++k) {
       mark();
       if (p1 > p0 && fused)
         k_ens_res_bres_owner<<<std::min(p1 - p0, cap[1]), blk[1], res_lds, st>>>(
@@ -743,18 +779,18 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
       if (t1 > t0)
         (k ? k_chain1 : k_chain0)<<<std::min(t1 - t0, cap[3 * k]), blk[3 * k], 0, st>>>(
             d_x, d_qold, d_q, d_res, d_adt, d_cell, d_crow, d_cbase, d_tiles, d_coff, t0, t1,
-            d_psum, d_pmax, d_ploc, S_at(off_chain[k]));
+            parts, S_at(off_chain[k]));
       mark();
     }
-    k_ens_finish<<<mhi - mlo, 256, 0, st>>>(d_psum, d_pmax, d_ploc, d_mtoff, mlo, d_slots,
+    k_ens_finish<<<mhi - mlo, 256, 0, st>>>(parts, half ? d_mblk : d_mtoff, half ? 1 : kGroups,
+                                            mlo, M, d_hist, d_count, d_done, capacity,
                                             S_at(off_fin));
   };
-  auto history = [&]() {
-    k_ens_history<<<1, 256, 0, st>>>(d_slots, hist_words, d_hist, d_count, capacity);
-  };
-
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
+  // graphs of one step and of kGraphSteps (launched where as many steps are
+  // left before the timed region or the end: a launch's gap on the device is
+  // paid once per graph)
+  hipGraph_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t gexec[2] = {nullptr, nullptr};
   std::vector<hipEvent_t> ev_a, ev_b;
   std::vector<double> member_ms(M, 0.0);
   int timed_steps = 0;
@@ -771,7 +807,8 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
   // candidate's time is its faster step (its launches in the step summed),
   // and the fastest candidate wins
   const int cand[5] = {64, 128, 256, 512, 1024};
-  const int ntune = (o->batched && o->autotune) ? std::min(10, o->niter) : 0;
+  // (nothing to tune for half steps: the patch fixes their workgroups)
+  const int ntune = (o->batched && o->autotune && !half) ? std::min(10, o->niter) : 0;
   double tune_ms[4][5];
   for (auto &row : tune_ms)
     for (double &v : row) v = INFINITY;
@@ -792,7 +829,6 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
       blk[0] = blk[2] = blk[3] = cand[ci];
       set_caps();
       step_range(0, M, tev);
-      history();
       ECHECK(hipStreamSynchronize(st));
       // event pairs: (res, bres, chain) twice
       const int kind[6] = {1, 2, 0, 1, 2, 3};
@@ -815,17 +851,18 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
       }
     } else if (o->batched) {
       if (o->graphed) {
-        if (!gexec) {
+        const int left = (it <= o->warmup ? o->warmup : o->niter) - it + 1;
+        const int k = left >= kGraphSteps, steps = k ? kGraphSteps : 1;
+        if (!gexec[k]) {
           ECHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-          step_range(0, M);
-          history();
-          ECHECK(hipStreamEndCapture(st, &graph));
-          ECHECK(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
+          for (int i = 0; i < steps; ++i) step_range(0, M);
+          ECHECK(hipStreamEndCapture(st, &graph[k]));
+          ECHECK(hipGraphInstantiate(&gexec[k], graph[k], nullptr, nullptr, 0));
         }
-        ECHECK(hipGraphLaunch(gexec, st));
+        ECHECK(hipGraphLaunch(gexec[k], st));
+        it += steps - 1;
       } else {
         step_range(0, M);
-        history();
       }
     } else {
       for (int m = 0; m < M; ++m) {
@@ -833,7 +870,6 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
         step_range(m, m + 1);
         if (o->member_timing) ECHECK(hipEventRecord(ev_b[m], st));
       }
-      history();
       if (o->member_timing && it > o->warmup) {
         ECHECK(hipStreamSynchronize(st));
         for (int m = 0; m < M; ++m) {
@@ -887,9 +923,9 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
     };
     const std::vector<int> no_items(M + 1, 0);  // bres_calc fused: no items of its own
     const std::vector<int> *bmoff = fused ? &no_items : &mesh_bitem_off;
-    const Seg segs[7] = {{off_res[0], &mblk},          {off_bres[0], bmoff},
-                         {off_chain[0], &mesh_tile_off}, {off_res[1], &mblk},
-                         {off_bres[1], bmoff},           {off_chain[1], &mesh_tile_off},
+    const std::vector<int> *ctoff = half ? &no_items : &mesh_tile_off;
+    const Seg segs[7] = {{off_res[0], &mblk},  {off_bres[0], bmoff}, {off_chain[0], ctoff},
+                         {off_res[1], &mblk},  {off_bres[1], bmoff}, {off_chain[1], ctoff},
                          {off_fin, nullptr}};
     std::vector<double> lat(M, 0.0);
     for (int it = o->warmup; it < o->niter; ++it) {
@@ -937,8 +973,10 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
   res->dead_res = dead ? 1 : 0;
   if (ntune)
     for (auto e : tev) (void)hipEventDestroy(e);
-  if (gexec) (void)hipGraphExecDestroy(gexec);
-  if (graph) (void)hipGraphDestroy(graph);
+  for (auto g : gexec)
+    if (g) (void)hipGraphExecDestroy(g);
+  for (auto g : graph)
+    if (g) (void)hipGraphDestroy(g);
   for (auto e : ev_a) (void)hipEventDestroy(e);
   for (auto e : ev_b) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(st);
