@@ -1071,6 +1071,81 @@ __global__ void __launch_bounds__(1024)
   op2h_red::write_partial(acc, parts, blockIdx.x);
 }
 
+// The boundary edges of each owned cell (at position pos[cell] of the owned
+// list, -1: not owned), up to four, in any order.  *bad: an edge of an unowned
+// cell, or a fifth of one cell.
+__global__ void k_bnd_edges(const int *__restrict becell, int n, const int *__restrict pos,
+                            int *__restrict cnt, int4 *slots, int *bad) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n) return;
+  const int i = pos[becell[e]];
+  const int k = i >= 0 ? atomicAdd(&cnt[i], 1) : 4;
+  if (k < 4) reinterpret_cast<int *>(slots)[4 * (size_t)i + k] = e;
+  else *bad = 1;
+}
+
+// Boundary edges of each block's owned cells.
+__global__ void __launch_bounds__(256)
+    k_bnd_totals(const int *__restrict owned_offs, const int *__restrict cnt,
+                 int *__restrict total) {
+  __shared__ int s;
+  const int b = blockIdx.x;
+  if (threadIdx.x == 0) s = 0;
+  __syncthreads();
+  int n = 0;
+  for (int i = owned_offs[b] + threadIdx.x; i < owned_offs[b + 1]; i += 256) n += cnt[i];
+  if (n) atomicAdd(&s, n);
+  __syncthreads();
+  if (threadIdx.x == 0) total[b] = s;
+}
+
+// Each owned cell's record: its interior increments (csr4), then its boundary
+// edges in order (of `key` when given: the application's) as 0x8000 | j, j
+// counting the block's boundary edges in owned order; edges[offs[b] + j] names
+// them.  *bad: more than four entries of a cell, or too many j.
+__global__ void __launch_bounds__(256)
+    k_bnd_records(const int *__restrict owned_offs, const ushort4 *__restrict csr4,
+                  const int *__restrict cnt, const int4 *__restrict slots,
+                  const int *__restrict key, const int *__restrict offs,
+                  ushort4 *__restrict rec, int *__restrict edges, int *bad) {
+  __shared__ int part[256];
+  const int b = blockIdx.x, t = threadIdx.x;
+  const int o0 = owned_offs[b], no = owned_offs[b + 1] - o0;
+  const int per = (no + 255) / 256, lo = min(no, t * per), hi = min(no, lo + per);
+  int n = 0;
+  for (int i = lo; i < hi; ++i) n += cnt[o0 + i];
+  part[t] = n;
+  __syncthreads();
+  int j = 0;
+  for (int i = 0; i < t; ++i) j += part[i];
+  for (int i = lo; i < hi; ++i) {
+    const ushort4 c = csr4[o0 + i];
+    unsigned short ent[4] = {c.x, c.y, c.z, c.w};
+    const int m = min(cnt[o0 + i], 4);
+    if (m) {
+      const int4 s4 = slots[o0 + i];
+      int e[4] = {s4.x, s4.y, s4.z, s4.w}, k = 0;
+      while (k < 4 && ent[k] != 0xFFFF) ++k;
+      auto before = [&](int x, int y) { return key ? key[x] < key[y] : x < y; };
+      for (int p = 1; p < m; ++p) {
+        const int v = e[p];
+        int q = p;
+        for (; q > 0 && before(v, e[q - 1]); --q) e[q] = e[q - 1];
+        e[q] = v;
+      }
+      for (int p = 0; p < m; ++p, ++j, ++k) {
+        if (k >= 4 || j >= 0x7FFF) {
+          *bad = 1;
+          break;
+        }
+        ent[k] = (unsigned short)(0x8000 | j);
+        edges[offs[b] + j] = e[p];
+      }
+    }
+    rec[o0 + i] = make_ushort4(ent[0], ent[1], ent[2], ent[3]);
+  }
+}
+
 // Rows of a four-node map as 16-bit offsets from the lowest node of their
 // 64-cell group, one wave per group; *wide is set where a group's nodes span
 // more than 65535.
@@ -1427,7 +1502,7 @@ void flush_res(void *) { launch_recorded(false, false, true); }
 void flush_halves(void *) { launch_recorded(false, false, false); }
 
 // The fused res_calc + bres_calc records for an owner plan and the boundary
-// map (bedge -> cell), built on the host once per plan: each owned cell's
+// map (bedge -> cell), built on the device once per plan: each owned cell's
 // interior increments, then its boundary edges (ascending; under transparent
 // renumbering in the application's order).  Null when a cell has more than
 // four increments in all, or the local ids do not fit 15 bits.
@@ -1455,60 +1530,44 @@ const BoundaryArgs *boundary_args(const op2h_owner_plan *p, op_map pbecell, op_m
   slot = BoundaryRec();
   slot.epoch = op2h_plan_epoch();
   if (!p->csr4 || pbecell->dim != 1 || (long long)p->max_elems * p->ninc >= 0x8000) return nullptr;
-  const int nb = p->nblocks, no = p->n_owned;
-  std::vector<int> oo(nb + 1), ow(std::max(no, 1)), eo(nb + 1), el(std::max(p->total, 1)),
-      co(no + 1);
-  op2h_owner_plan_download(p, oo.data(), ow.data(), eo.data(), el.data(), co.data(), nullptr);
-  std::vector<unsigned short> csr(std::max(co[no], 1));
-  op2h_owner_plan_download(p, nullptr, nullptr, nullptr, nullptr, nullptr, csr.data());
-  // boundary edges per cell, in order
-  const int nbe = pbecell->from->size, ncell = p->to_size;
-  const int *key_be = op2h::old_index_host(pbecell->from);
-  const int *becell = op2h::host_map(pbecell);  // in the device numbering
-  std::vector<int> bo(ncell + 1, 0), order(nbe);
-  for (int e = 0; e < nbe; ++e) bo[becell[e] + 1]++;
-  for (int c = 0; c < ncell; ++c) bo[c + 1] += bo[c];
-  for (int e = 0; e < nbe; ++e) order[e] = e;
-  if (key_be)
-    std::sort(order.begin(), order.end(), [&](int a, int b) { return key_be[a] < key_be[b]; });
-  std::vector<int> fill(bo.begin(), bo.end() - 1), bl(std::max(nbe, 1));
-  for (int e : order) bl[fill[becell[e]]++] = e;
-  std::vector<ushort4> rec(std::max(no, 1));
-  std::vector<int> offs(nb + 1, 0), edges;
-  for (int b = 0; b < nb; ++b) {
-    offs[b] = (int)edges.size();
-    for (int i = oo[b]; i < oo[b + 1]; ++i) {
-      unsigned short ent[4] = {0xFFFF, 0xFFFF, 0xFFFF, 0xFFFF};
-      int k = 0;
-      for (int j = co[i]; j < co[i + 1]; ++j) {
-        if (k == 4) return nullptr;
-        ent[k++] = csr[j];
-      }
-      const int cell = ow[i];
-      for (int j = bo[cell]; j < bo[cell + 1]; ++j) {
-        const int local = (int)edges.size() - offs[b];
-        if (k == 4 || local >= 0x7FFF) return nullptr;
-        ent[k++] = (unsigned short)(0x8000 | local);
-        edges.push_back(bl[j]);
-      }
-      rec[i] = make_ushort4(ent[0], ent[1], ent[2], ent[3]);
-    }
-  }
-  offs[nb] = (int)edges.size();
-  if (edges.size() != (size_t)nbe) return nullptr;  // a boundary edge of an unowned cell
+  const int nb = p->nblocks, no = p->n_owned, ncell = p->to_size;
+  const int nbe = pbecell->from->size;
+  if (!nb) return nullptr;
   char name[96];
   snprintf(name, sizeof name, "res_bres.fused.%p.%d", (const void *)p, pbecell->index);
   const size_t b_rec = ((size_t)8 * std::max(no, 1) + 255) / 256 * 256;
   const size_t b_offs = ((size_t)4 * (nb + 1) + 255) / 256 * 256;
   int fresh = 0;
-  char *buf = (char *)op2h_plan_user(name, b_rec + b_offs + 4 * std::max<size_t>(edges.size(), 1),
-                                     &fresh);
-  KCHECK(hipMemcpyAsync(buf, rec.data(), 8 * (size_t)no, hipMemcpyHostToDevice, st));
-  KCHECK(hipMemcpyAsync(buf + b_rec, offs.data(), 4 * (size_t)(nb + 1), hipMemcpyHostToDevice, st));
-  if (!edges.empty())
-    KCHECK(hipMemcpyAsync(buf + b_rec + b_offs, edges.data(), 4 * edges.size(),
-                          hipMemcpyHostToDevice, st));
+  char *buf = (char *)op2h_plan_user(name, b_rec + b_offs + 4 * (size_t)std::max(nbe, 1), &fresh);
+  // scratch: each owned cell's boundary edges and their number, each cell's
+  // position, each block's number, the flag
+  const size_t b_slots = (size_t)16 * no, b_cnt = (size_t)4 * no, b_pos = (size_t)4 * ncell;
+  char *tmp = nullptr;
+  KCHECK(hipMalloc(&tmp, b_slots + b_cnt + b_pos + 4 * (size_t)nb + 4));
+  int4 *slots = (int4 *)tmp;
+  int *cnt = (int *)(tmp + b_slots), *pos = (int *)(tmp + b_slots + b_cnt);
+  int *total = (int *)(tmp + b_slots + b_cnt + b_pos), *bad = total + nb;
+  KCHECK(hipMemsetAsync(cnt, 0, b_cnt, st));
+  KCHECK(hipMemsetAsync(pos, 0xFF, b_pos, st));
+  KCHECK(hipMemsetAsync(bad, 0, 4, st));
+  k_patch_pos<<<grid_for(no, 256), 256, 0, st>>>(p->owned, no, pos);
+  if (nbe)
+    k_bnd_edges<<<grid_for(nbe, 256), 256, 0, st>>>(pbecell->map_d, nbe, pos, cnt, slots, bad);
+  k_bnd_totals<<<nb, 256, 0, st>>>(p->owned_offs, cnt, total);
+  std::vector<int> offs((size_t)nb + 1, 0);
+  KCHECK(hipMemcpyAsync(offs.data() + 1, total, 4 * (size_t)nb, hipMemcpyDeviceToHost, st));
   KCHECK(hipStreamSynchronize(st));
+  for (int b = 0; b < nb; ++b) offs[b + 1] += offs[b];
+  KCHECK(hipMemcpyAsync(buf + b_rec, offs.data(), 4 * ((size_t)nb + 1), hipMemcpyHostToDevice, st));
+  k_bnd_records<<<nb, 256, 0, st>>>(p->owned_offs, (const ushort4 *)p->csr4, cnt, slots,
+                                    op2h_set_old_index(pbecell->from), (const int *)(buf + b_rec),
+                                    (ushort4 *)buf, (int *)(buf + b_rec + b_offs), bad);
+  KCHECK(hipGetLastError());
+  int failed = 0;
+  KCHECK(hipMemcpyAsync(&failed, bad, 4, hipMemcpyDeviceToHost, st));
+  KCHECK(hipStreamSynchronize(st));
+  KCHECK(hipFree(tmp));
+  if (failed) return nullptr;
   BoundaryArgs &B = slot.B;
   B.rec = (const ushort4 *)buf;
   B.offs = (const int *)(buf + b_rec);

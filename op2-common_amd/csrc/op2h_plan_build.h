@@ -112,6 +112,27 @@ bool owner_lists(int nto, int nel, int dim, const int *map, int ninc,
                  std::string &err, const int *elem_key = nullptr,
                  bool key_instances = true);
 
+// The graph the patches are grown over: target t's neighbours adj[off[t],
+// off[t + 1]) in element order, whether any element names t, and the widest
+// spread of one element's targets.
+struct TargetGraph {
+  std::vector<int> off, adj;
+  std::vector<char> used;
+  long long width = 0;
+};
+
+// The same on the device (op2h_owner_gpu.hip), from the increment map's device
+// table: the graph, and a plan's lists for patches grown over it (false, and
+// the record's lists unset, when a block or a target's list is too long for
+// it; blocks until built).  gpu_owner_fits: whether the loop's shape is theirs.
+bool gpu_owner_fits(int nto, int nel, int ninc);
+void gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc,
+                      const int *inc_idx, hipStream_t stream, TargetGraph &g);
+bool gpu_owner_lists(int nto, int nel, int dim, const int *map_d, int ninc,
+                     const int *inc_idx, int nb, const std::vector<int> &block_of,
+                     const int *elem_key, bool key_instances, hipStream_t stream,
+                     OwnerPlanRec &rec);
+
 std::unique_ptr<OwnerPlanRec> build_owner_plan(op_set set, int block_cells,
                                                int nargs, const op_arg *args,
                                                hipStream_t stream,
