@@ -131,6 +131,11 @@ int op2h_dat_soa_stride(op_dat dat);
  * The kernel writes the loop's own reduction over the set (identity-started)
  * into the slot; op2h_loop_end combines it with the host value. */
 void *op2h_gbl_slot(op2h_loop_ctx *ctx, int argi, int info_argi);
+/* The same for a kernel that only stores its result, once: outside capture the
+ * pinned host memory that op2h_loop_end reads, so that no copy follows the
+ * kernel (two copies after every airfoil update took 12 of its 30 us at 59,000
+ * cells). */
+void *op2h_gbl_result(op2h_loop_ctx *ctx, int argi, int info_argi);
 
 /* Deferred gbl reductions inside a captured graph.  A stub that reduces a
  * dim-1 double gbl arg through per-workgroup partials may, while a graph is

@@ -2231,8 +2231,8 @@ extern "C" void op_par_loop_airfoil_5_update(char const *name, op_set set,
   }
   if (!deferred) {
     if (!g_halves.empty()) flush_halves(nullptr);
-    slot_rms = (double *)op2h_gbl_slot(&ctx, 4, -1);
-    slot_max = (double *)op2h_gbl_slot(&ctx, 5, 7);
+    slot_rms = (double *)op2h_gbl_result(&ctx, 4, -1);
+    slot_max = (double *)op2h_gbl_result(&ctx, 5, 7);
     parts = update_parts(op2h_reduct_scratch((size_t)g * kPartBytes), g);
   }
   if (is_float(args[2]) != is_float(args[3])) {

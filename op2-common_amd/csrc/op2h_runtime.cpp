@@ -1908,7 +1908,7 @@ extern "C" void op2h_loop_end(op2h_loop_ctx *ctx) {
     size_t bytes = (size_t)a.size + (with_info ? ctx->args[info].size : 0);
     // inside a captured graph the slots reach the host through the history
     // record of the launch (no per-loop copy node)
-    if (!R.capturing)
+    if (!R.capturing && ctx->gbl_slot_d[g] != ctx->gbl_slot_h[g])
       HIPCHECK(hipMemcpyAsync(ctx->gbl_slot_h[g], ctx->gbl_slot_d[g], bytes,
                               hipMemcpyDeviceToHost, R.stream));
     if (R.capturing) {
@@ -2015,6 +2015,13 @@ extern "C" void *op2h_gbl_slot(op2h_loop_ctx *ctx, int argi, int info_argi) {
   ctx->gbl_slot_d[g] = slot.first;
   ctx->gbl_slot_h[g] = slot.second;
   return slot.first;
+}
+
+extern "C" void *op2h_gbl_result(op2h_loop_ctx *ctx, int argi, int info_argi) {
+  void *slot = op2h_gbl_slot(ctx, argi, info_argi);
+  if (rt().capturing) return slot;  // the history record reads it on the device
+  const int g = ctx->ngbl - 1;
+  return ctx->gbl_slot_d[g] = ctx->gbl_slot_h[g];  // nothing to copy in op2h_loop_end
 }
 
 namespace {

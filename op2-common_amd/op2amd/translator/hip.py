@@ -649,7 +649,7 @@ class LoopGen:
         s.append(f"                    nullptr, 0, set->size, 1, partials, 0, step);")
         s.append(f"    }}")
         if self.reds:
-            slots = ", ".join(f"(unsigned char *)op2h_gbl_slot(&ctx, {j}, {self.info_of.get(j, -1)})"
+            slots = ", ".join(f"(unsigned char *)op2h_gbl_result(&ctx, {j}, {self.info_of.get(j, -1)})"
                               for j in self.reds)
             # one workgroup of 256: at most 2048 records (8 per thread) outside
             # colouring; fewer waves make its barriers and wave combines cheaper
