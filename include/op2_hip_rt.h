@@ -143,10 +143,9 @@ void *op2h_gbl_result(op2h_loop_ctx *ctx, int argi, int info_argi);
  * them: op2h_gbl_partials returns 1 with device buffers for `nparts`
  * partials, vals[nparts] and, for OP_MIN/OP_MAX with a linked dim-1 int info
  * arg, locs[nparts] (the info payload, which must be the element index: equal
- * values keep the lowest).  The graph's history kernel then combines them in
- * partial order (thread t takes partials t and t + 1024, then wave trees, then
- * the 16 waves in order) when it records the launch, so one kernel finishes
- * every deferred reduction of a step.  Outside capture it returns 0 with
+ * values keep the lowest).  The graph's history kernel then combines them in a
+ * fixed order (group_reduce of op2h_reduce.h) when it records the launch, so
+ * one kernel finishes every deferred reduction of a step.  Outside capture it returns 0 with
  * NULLs, and the stub finishes the reduction into op2h_gbl_slot itself. */
 int op2h_gbl_partials(op2h_loop_ctx *ctx, int argi, int info_argi, int nparts,
                       double **vals, int **locs);

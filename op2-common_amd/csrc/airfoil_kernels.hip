@@ -7,14 +7,18 @@
 // device functions with the reference's expression trees; the whole library is
 // compiled with -ffp-contract=off, so each multiply and add rounds as in the
 // reference's host build.  Loops with indirect increments (res_calc,
-// bres_calc) have four plans:
+// bres_calc) have five plans:
 //   ATOMIC  one thread per edge, FP64 atomics on res;
 //   COLOR   flat colouring, one launch per colour, plain read-modify-write;
 //   STAGED  plan blocks staged in LDS, increments applied colour by colour
 //           inside the block, blocks launched colour by colour;
 //   GATHER  one thread per cell, the edges of the cell visited in edge order
 //           and res accumulated in registers — the sequential executor's
-//           summation order, so results match it bit for bit.
+//           summation order, so results match it bit for bit;
+//   OWNER   one workgroup per patch of cells, each edge's flux once per patch
+//           into LDS, each cell summing its own in edge order: the same bits.
+// Inside a captured graph whole half steps run as one launch each
+// (airfoil_patch.h).
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 

@@ -1,13 +1,13 @@
 // Batched airfoil ensembles (include/op2amd_ensemble.h).
 //
-// Members are concatenated into one mesh; every loop of the time step is one
-// persistent launch over all members' work items (runs of one member's
-// elements, found through per-member offset tables), except in the looped
-// baseline, which launches each loop once per member over that member's
-// items.  res_calc and bres_calc use the owner-compute plan (each cell sums
-// its edges' fluxes in edge order), and the reductions' partials are formed
-// per tile, so results do not depend on the launch structure or the
-// workgroup sizes.
+// Members are concatenated into one mesh; each half step is one persistent
+// launch over all members' patches (half_step_patch), or, with bres_calc kept
+// apart or patches too large for it, each loop one over all members' work items
+// (runs of one member's elements, found through per-member offset tables).  The
+// looped baseline launches once per member over that member's items.  Every
+// cell sums its edges' fluxes in edge order and the reductions are pair sums
+// (Sum2), so results do not depend on the launch structure or the workgroup
+// sizes.
 #include "op2amd_ensemble.h"
 
 #include <hip/hip_runtime.h>
