@@ -1420,11 +1420,11 @@ void launch_half_as(const Half &h, const HalfArgs<R> &H, const PendingDirect &D)
 // The time step of halves h and k as two launches (is_step holds).  D: the
 // second update; adt: an adt_calc follows it; dead_save: the next time step is
 // run the same way, so nothing reads the copy of q that D's save_soln would
-// make, nor was this step's own copy made when saved is false; zeroed: res
-// holds zeros in memory.
+// make, nor was this step's own copy made when saved is false.  res holds zeros
+// in memory where h.R.zero says so (the update before zeroed this very res).
 template <class R>
 void launch_step_as(const Half &h, const Half &k, const PendingDirect &D, bool adt,
-                    bool dead_save, bool saved, bool zeroed) {
+                    bool dead_save, bool saved) {
   const HalfMem &M = g_half_mem;
   double *q = const_cast<double *>(h.R.q), *qold = h.C.P.save_dst;
   R *a = (R *)const_cast<void *>(h.R.adt), *a2 = (R *)M.adt2;
@@ -1440,7 +1440,7 @@ void launch_step_as(const Half &h, const Half &k, const PendingDirect &D, bool a
   H.oldidx = k.C.P.oldidx;
   H.sx = h.R.sx;
   H.sq = h.R.sq;
-  H.flags = kHalfAdt | (zeroed ? 0 : kHalfReadRes | kHalfZeroRes);
+  H.flags = kHalfAdt | (h.R.zero ? 0 : kHalfReadRes | kHalfZeroRes);
   launch_half_as<R>(h, H, k.C.P);
   H.q = M.q2;
   H.adt = a2;
@@ -1478,13 +1478,12 @@ void launch_recorded(bool direct, bool chain, bool res) {
   for (int i = 0; i < n;) {
     if (step_at(i)) {
       if (!folded) launch_chain(hs[i].C, false);
-      const bool zeroed = folded || hs[i].C.P.upd;
       const PendingDirect *d;
       const PendingChain *c;
       follows(i + 1, &d, &c);
       const bool dead = c && d->save && step_at(i + 2);
-      if (hs[i].R.mixed) launch_step_as<float>(hs[i], hs[i + 1], *d, c, dead, saved, zeroed);
-      else launch_step_as<double>(hs[i], hs[i + 1], *d, c, dead, saved, zeroed);
+      if (hs[i].R.mixed) launch_step_as<float>(hs[i], hs[i + 1], *d, c, dead, saved);
+      else launch_step_as<double>(hs[i], hs[i + 1], *d, c, dead, saved);
       folded = true;
       saved = !dead;
       i += 2;

@@ -125,6 +125,47 @@ def test_captured_sequences_leave_every_dat_as_eager_loops_do(name, soa):
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("names", ["two steps", "an update, then a step"])
+def test_steps_on_another_res_read_and_zero_it(names):
+    """Captured steps that increment a second res dat, which holds values: the
+    update before them zeroed the first one, so its zeros say nothing here."""
+    mesh = op2amd.mesh.generate(70, 41, 2, "rcm")
+    q, res = inputs(mesh, 4)
+
+    def run(captured):
+        app = Program(mesh, q, res)
+        try:
+            first, second = app.res, api.decl_dat(app.cells, 4, "double", 2 * res, "p_res2")
+
+            def play():
+                app.res = first
+                app.play(STEP if names == "two steps" else ["update"])
+                app.res = second
+                app.play(STEP)
+            api.op2h_set_sync_mode(api.SYNC_GBL_ONLY)
+            api.op2h_set_loop_plan(b"res_calc", api.PLAN_OWNER, 128)
+            api.op2h_set_loop_plan(b"bres_calc", api.PLAN_GATHER, 128)
+            for app.res in (second, first):  # builds the plans; both hold values again
+                app.play(STEP[:-1])
+            if captured:
+                assert api.lib.op2h_graph_begin() == 0
+                play()
+                assert api.lib.op2h_graph_end() == 0
+                assert api.lib.op2h_graph_launch(1) == 0
+                api.op2h_device_sync()
+            else:
+                play()
+            app.res = first
+            out = app.state()
+            app.res = second
+            return out + app.state()
+        finally:
+            app.close()
+
+    for a, b in zip(run(False), run(True)):
+        assert np.array_equal(a, b)
+
+
 def test_update_reductions_do_not_depend_on_the_grouping():
     """rms is a sum of unevaluated pairs rounded once: the same bits for every
     workgroup size and launch shape, within 2^-52 of the exactly rounded sum
