@@ -137,6 +137,14 @@ struct UpdateAcc {
   MaxLoc ml{-INFINITY, 0x7fffffff};
 };
 
+// One cell's share, its sum and its own maximum: joined as any other maximum,
+// because the cells a thread takes need not come in index order (a thread's
+// running maximum would keep the first it visits of two equal ones).
+__device__ __forceinline__ void add_cell(UpdateAcc &a, double sum, MaxLoc ml) {
+  sum2_add(a.rms, sum);
+  a.ml = maxloc_combine(a.ml, ml);
+}
+
 __device__ __forceinline__ void wave_join(UpdateAcc &a) {
   for (int o = 32; o > 0; o >>= 1) {
     a.rms = sum2_join(a.rms, Sum2{__shfl_xor(a.rms.hi, o, 64), __shfl_xor(a.rms.lo, o, 64)});

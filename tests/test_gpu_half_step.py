@@ -166,6 +166,45 @@ def test_steps_on_another_res_read_and_zero_it(names):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("names", [["update"], ["update", "save_soln", "adt_calc"], STEP],
+                         ids=["eager update", "direct chain", "half steps"])
+def test_equal_maxima_keep_the_lowest_application_index(names):
+    """288,000 renumbered cells (two and more per thread of every form of the
+    update) of which all from one on have exactly the same change: at rest on a
+    uniform mesh with sides that are powers of two every flux of mass is zero
+    and pressures cancel exactly, so their res is what they start with."""
+    mesh = op2amd.mesh.generate(640, 450, 5, "random")  # (the nodes stay in rows)
+    mesh.x[:] = np.stack(np.divmod(np.arange(mesh.nnode), 641)[::-1], 1) * 2.0 ** -9
+    mesh.bound[:] = 1
+    q = np.tile([1.0, 0.0, 0.0, 2.5], (mesh.ncell, 1))
+    captured = len(names) > 1
+    for first in (0, 1, 2, 3, 5, 8, 20):
+        res = np.zeros((mesh.ncell, 4))
+        res[first:, 0] = 2.0 ** -10
+        app = Program(mesh, q, res, tokens=("OP_HIP_RENUMBER",))
+        try:
+            api.op2h_set_sync_mode(api.SYNC_GBL_ONLY)
+            api.op2h_set_loop_plan(b"res_calc", api.PLAN_OWNER, 64)
+            api.op2h_set_loop_plan(b"bres_calc", api.PLAN_GATHER, 128)
+            app.play(["adt_calc", "res_calc", "bres_calc"])  # builds the plans
+            if captured:
+                assert api.lib.op2h_graph_begin() == 0
+                app.play(names)
+                assert api.lib.op2h_graph_end() == 0
+                assert api.lib.op2h_graph_launch(1) == 0
+                record, n = np.zeros(6), C.c_int()
+                api.lib.op2h_graph_history(1, record.ctypes.data_as(C.c_void_p), C.byref(n))
+                assert record[1] > 0
+                at = int(record.view(np.int32)[4])
+            else:
+                rms, maxerr, errloc = C.c_double(), C.c_double(), C.c_int(-1)
+                app.update(rms, maxerr, errloc)
+                at = errloc.value
+            assert at == first
+        finally:
+            app.close()
+
+
 def test_update_reductions_do_not_depend_on_the_grouping():
     """rms is a sum of unevaluated pairs rounded once: the same bits for every
     workgroup size and launch shape, within 2^-52 of the exactly rounded sum

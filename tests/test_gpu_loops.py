@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 class App:
     """Declares the airfoil sets/maps/dats through the OP2 C API."""
 
-    def __init__(self, mesh, q, res, soa=False):
-        api.init(*(["OP_AUTO_SOA"] if soa else []))
+    def __init__(self, mesh, q, res, soa=False, tokens=()):
+        api.init(*tokens, *(["OP_AUTO_SOA"] if soa else []))
         self.m = mesh
         self.nodes = api.op_decl_set(mesh.nnode, b"nodes")
         self.edges = api.op_decl_set(mesh.nedge, b"edges")
