@@ -89,7 +89,8 @@ __global__ void k_neighbours(Map m, const int *__restrict off, int *__restrict f
   }
 }
 
-// Each target's neighbours in element order, as targets.
+// Each target's neighbours (at most kListMax (ninc - 1)) in element order, as
+// targets.
 __global__ void k_order_neighbours(Map m, const int *__restrict off,
                                    unsigned long long *__restrict adj, int *__restrict out) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -297,7 +298,7 @@ bool gpu_owner_fits(int nto, int nel, int ninc) {
   return ninc <= kMaxInc && (long long)nel * ninc * ninc <= INT_MAX && nto > 0;
 }
 
-void gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc, const int *inc_idx,
+bool gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc, const int *inc_idx,
                       hipStream_t st, TargetGraph &g) {
   Scratch S;
   const Map m = map_of(nto, nel, dim, map_d, ninc, inc_idx);
@@ -312,11 +313,15 @@ void gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc, con
   OGCHECK(hipMemcpyAsync(&w, width, sizeof w, hipMemcpyDeviceToHost, st));
   OGCHECK(hipStreamSynchronize(st));
   g.width = w;
+  // a target that so many elements name has more increments than its list here
+  // may hold, and ordering its neighbours would be one thread's work
+  for (int t = 0; t < nto; ++t)
+    if (g.off[t + 1] > kListMax * (ninc - 1)) return false;
   g.off[0] = 0;
   for (int t = 0; t < nto; ++t) g.off[t + 1] += g.off[t];
   const size_t n = g.off[nto];
   g.adj.resize(n);
-  if (!n) return;
+  if (!n) return true;
   int *off = S.get<int>((size_t)nto + 1, false, st), *out = S.get<int>(n, false, st);
   unsigned long long *adj = S.get<unsigned long long>(n, false, st);
   OGCHECK(hipMemcpyAsync(off, g.off.data(), sizeof(int) * ((size_t)nto + 1),
@@ -327,6 +332,7 @@ void gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc, con
   OGCHECK(hipGetLastError());
   OGCHECK(hipMemcpyAsync(g.adj.data(), out, sizeof(int) * n, hipMemcpyDeviceToHost, st));
   OGCHECK(hipStreamSynchronize(st));
+  return true;
 }
 
 bool gpu_owner_lists(int nto, int nel, int dim, const int *map_d, int ninc, const int *inc_idx,

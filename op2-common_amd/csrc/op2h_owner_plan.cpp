@@ -316,9 +316,9 @@ std::unique_ptr<OwnerPlanRec> build_owner_plan(op_set set, int block_cells,
   P.block_cells = block_cells;
   P.ninc = ninc;
   // large loops have their lists built on the device, where they fit
-  if (nel >= kDeviceLists && gpu_owner_fits(nto, nel, ninc)) {
-    TargetGraph g;
-    gpu_target_graph(nto, nel, dim, own->map_d, ninc, inc_idx.data(), stream, g);
+  TargetGraph g;
+  if (nel >= kDeviceLists && gpu_owner_fits(nto, nel, ninc) &&
+      gpu_target_graph(nto, nel, dim, own->map_d, ninc, inc_idx.data(), stream, g)) {
     std::vector<int> block_of;
     const int nb = grow_over(nto, g, block_cells, block_of);
     if (gpu_owner_lists(nto, nel, dim, own->map_d, ninc, inc_idx.data(), nb, block_of,

@@ -122,11 +122,13 @@ struct TargetGraph {
 };
 
 // The same on the device (op2h_owner_gpu.hip), from the increment map's device
-// table: the graph, and a plan's lists for patches grown over it (false, and
-// the record's lists unset, when a block or a target's list is too long for
-// it; blocks until built).  gpu_owner_fits: whether the loop's shape is theirs.
+// table: the graph (false, and the graph unset, when a target has more
+// neighbours than a list could hold), and a plan's lists for patches grown over
+// it (false, and the record's lists unset, when a block or a target's list is
+// too long for it); both block until built.  gpu_owner_fits: whether the loop's
+// shape is theirs.
 bool gpu_owner_fits(int nto, int nel, int ninc);
-void gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc,
+bool gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc,
                       const int *inc_idx, hipStream_t stream, TargetGraph &g);
 bool gpu_owner_lists(int nto, int nel, int dim, const int *map_d, int ninc,
                      const int *inc_idx, int nb, const std::vector<int> &block_of,

@@ -89,3 +89,29 @@ def test_targets_with_hundreds_of_increments_use_the_host_lists():
     p = plan_of(Star, 10)
     assert p.max_incs > 64 and p.n_owned == 100
     api.op_exit()
+
+
+@pytest.mark.parametrize("hub", [64, 65, 25000])
+def test_a_target_that_many_elements_name(hub):
+    """30,000 elements of which `hub` name target 0: up to 64 of them the lists
+    are built on the device, beyond on the host, where a target's list costs
+    what it is long.  (In one thread's insertion sort 25,000 neighbours would
+    be about 10^8 dependent moves in memory, seconds; the host takes
+    milliseconds.)"""
+    n = 30000
+    ecell = np.stack([np.where(np.arange(n) % (n // hub) == 0, 0, 1 + np.arange(n)), 1 + n + np.arange(n)], 1).astype(np.int32)
+    ecell[np.flatnonzero(ecell[:, 0] == 0)[hub:], 0] = 1
+
+    class Star:
+        nedge, ncell = n, 2 * n + 1
+    Star.ecell = ecell
+    p = plan_of(Star, 64)
+    try:
+        assert p.max_incs == hub and p.build_ms < 1000
+        oo, ow, eo, el, co, cs = lists(p, n)
+    finally:
+        api.op_exit()
+    nb, block_of = api.owner_partition(Star.ncell, ecell, [0, 1], 64)
+    got = np.full(Star.ncell, -1, np.int32)
+    got[ow] = np.repeat(np.arange(nb), np.diff(oo))
+    assert p.nblocks == nb and np.array_equal(got, block_of)
