@@ -634,6 +634,9 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
                             &pa_nc, &pa_nn);
   const size_t half_lds = patch_lds_bytes<double>(pa_nc, pa_nn);
   half = half && half_lds <= 64 * 1024;
+  // whole waves: the reductions shuffle over 64 lanes, and the lanes past a
+  // patch's cells hold nothing
+  const int half_blk = (patch + 63) / 64 * 64;
   double *d_q2 = half ? dev_alloc<double>(4 * (size_t)Nc, keep) : nullptr;
   double *d_adt2 = half ? dev_alloc<double>(Nc, keep) : nullptr;
   std::vector<int2> pmember(npatch);
@@ -708,9 +711,9 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
     cap[2] = resident((const void *)k_ens_bres, blk[2], 0) * (blk[2] / 64);  // waves
     cap[3] = resident((const void *)k_chain1, blk[3], 0);
     if (half) {  // one launch per half step over the patches
-      blk[0] = blk[3] = patch;
-      cap[0] = resident((const void *)k_ens_half<false>, patch, half_lds);
-      cap[1] = cap[3] = resident((const void *)k_ens_half<true>, patch, half_lds);
+      blk[0] = blk[3] = half_blk;
+      cap[0] = resident((const void *)k_ens_half<false>, half_blk, half_lds);
+      cap[1] = cap[3] = resident((const void *)k_ens_half<true>, half_blk, half_lds);
     }
   };
   set_caps();
@@ -755,7 +758,7 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
       const int most = std::max(1, std::min(p1 - p0, cap[3 * k]));
       const int rounds = (p1 - p0 + most - 1) / most, grid = (p1 - p0 + rounds - 1) / std::max(1, rounds);
       if (p1 > p0)
-        (k ? k_ens_half<true> : k_ens_half<false>)<<<grid, patch, half_lds, st>>>(
+        (k ? k_ens_half<true> : k_ens_half<false>)<<<grid, half_blk, half_lds, st>>>(
             H, PA, BA, d_pmember, pa_nc, pa_nn, p0, p1, parts, S_at(off_res[k]));
     }
     for (int k = 0; k < 2 && !half; ++k) {

@@ -118,11 +118,11 @@ def test_bres_calc_fused_into_res_calc_gives_the_same_bits(max_workgroups):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("patch_cells", [64, 128, 1024])
+@pytest.mark.parametrize("patch_cells", [64, 65, 100, 128, 333, 1000, 1024])
 def test_res_calc_patch_size_changes_no_bits(patch_cells):
-    """Owner patches of 64, 128 or 1024 cells (one workgroup each) give the
-    bits of the default 256-cell patches: each cell sums its edges' fluxes in
-    edge order whatever patch holds it."""
+    """Owner patches of 64 to 1024 cells (one workgroup each), whole waves or
+    not, give the bits of the default 256-cell patches: each cell sums its
+    edges' fluxes in edge order whatever patch holds it."""
     sp = op2amd.ensemble.spec(nmesh=4, min_IJ=(40, 20), max_IJ=(160, 80), seed=7)
     ref = op2amd.ensemble.run(sp, 10, batched=True, graphed=True, want_q=True)
     run = op2amd.ensemble.run(sp, 10, batched=True, graphed=True, want_q=True,
