@@ -177,6 +177,15 @@ __device__ __forceinline__ void tiles_product(const float *a, const float *W, in
   for (; k < K; k += 4) steps(std::integral_constant<int, 1>());
 }
 
+// LDS written by a lane of this wave before and read by another after (or read
+// before and written after): the hardware keeps a wave's LDS accesses in order,
+// the fences make the compiler do so too.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 16 samples per wave: Y, and with BACK the samples' A1, A2, DY, D2 and D1,
 // which the weight gradients are formed from.  The parameters and the rows'
 // activations stay in LDS (25 KiB and 8.5 KiB a wave for the cost model's).  X and Y may be pinned
@@ -241,7 +250,7 @@ __global__ void __launch_bounds__(64 * kRowWaves)
       if (BACK && i0 + r4 + e < n) A1[(size_t)(i0 + r4 + e) * H + j] = a;
     }
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   tiles_product<NT>(v, w2, kRowStride, 1, H, lane, acc);
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -252,7 +261,7 @@ __global__ void __launch_bounds__(64 * kRowWaves)
       if (BACK && i0 + r4 + e < n) A2[(size_t)(i0 + r4 + e) * H + j] = a;
     }
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   // one output column: the other lanes' products (of W3's neighbours) are unused
   f32x4 y;
   tiles_product<1>(u, w3, 1, 0, H, lane, &y);
@@ -272,6 +281,7 @@ __global__ void __launch_bounds__(64 * kRowWaves)
   const float d0 = __shfl(dy[0], (lane & 12) << 2), d1 = __shfl(dy[1], (lane & 12) << 2),
               d2 = __shfl(dy[2], (lane & 12) << 2), d3 = __shfl(dy[3], (lane & 12) << 2);
   const float dr = (lane & 3) == 0 ? d0 : (lane & 3) == 1 ? d1 : (lane & 3) == 2 ? d2 : d3;
+  wave_sync();  // y's product has read u
   for (int t = 0; t < NT; ++t) {
     const int j = 16 * t + col;
     f32x4 d = {0.f, 0.f, 0.f, 0.f};
@@ -283,7 +293,7 @@ __global__ void __launch_bounds__(64 * kRowWaves)
       if (i0 + r4 + e < n) D2[(size_t)(i0 + r4 + e) * H + j] = *a;
     }
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   // D1 = (D2 W2^T) where A1 > 0
   tiles_product<NT>(u, w2, 1, kRowStride, H, lane, acc);
 #pragma unroll
