@@ -112,6 +112,9 @@ void op2h_set_streaming(int mode);
 int op2h_streaming(size_t stream_bytes);
 /* Pending launches taken over by a later stub since the library loaded. */
 unsigned long long op2h_fused_count(void);
+/* Half steps of the airfoil loops launched as one kernel each (into captured
+ * graphs) since the library loaded. */
+unsigned long long op2h_half_step_count(void);
 
 /* Called by op2h_graph_begin before the capture starts: a kernel file
  * allocates and packs there what its launches inside a capture need (nothing

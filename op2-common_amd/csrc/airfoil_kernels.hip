@@ -1361,6 +1361,7 @@ struct HalfMem {
   int nc = 0, nn = 0;
 };
 HalfMem g_half_mem;
+unsigned long long g_half_steps = 0;  // k_half_step launches
 
 // Whether halves h and k (with the direct loops D that follow k, and its
 // adt_calc C if that follows too) are one time step of the form
@@ -1417,6 +1418,7 @@ void launch_half_as(const Half &h, const HalfArgs<R> &H, const PendingDirect &D)
   op2h_gbl_partials_used(D.parts.mx, grid);
   launch_k(false, nullptr, nullptr, kern, grid, P.bs, lds, P.st, H, M.patches, h.B, npatch, M.nc,
            M.nn, D.parts);
+  ++g_half_steps;
 }
 
 // The time step of halves h and k as two launches (is_step holds).  D: the
@@ -1696,6 +1698,8 @@ const struct CaptureHook {
 } g_capture_hook;
 
 }  // namespace
+
+extern "C" unsigned long long op2h_half_step_count(void) { return g_half_steps; }
 
 extern "C" void op_par_loop_airfoil_1_save_soln(char const *name, op_set set,
                                                 op_arg arg0, op_arg arg1) {

@@ -19,24 +19,34 @@ KEYS = ("rms", "rms_k0", "maxerr", "errloc", "q")
 
 
 def fused_and_not(mesh, niter, **kw):
+    """The runs with and without fusion, and how many half steps the first
+    one's graph holds."""
     kw = dict(dict(mode="graphed", plan_res="owner", plan_bres="gather", graph_steps=4), **kw)
+    n0 = api.op2h_half_step_count()
     fused = op2amd.airfoil.run(mesh, niter, **kw)
+    n1 = api.op2h_half_step_count()
     api.op2h_set_fusion(0)
     try:
-        return fused, op2amd.airfoil.run(mesh, niter, **kw)
+        plain = op2amd.airfoil.run(mesh, niter, **kw)
     finally:
         api.op2h_set_fusion(1)
+    assert api.op2h_half_step_count() == n1
+    return fused, plain, n1 - n0
 
 
 @pytest.mark.parametrize("I,J,ordering,block", [
     (2, 2, "structured", 64), (9, 7, "structured", 64), (16, 8, "random", 128),
     (33, 31, "rcm", 64), (61, 47, "random", 192), (90, 90, "hilbert", 256),
-    (100, 83, "structured", 1024), (64, 64, "rcm", 512)])
+    (100, 83, "structured", 1024), (64, 64, "rcm", 512), (640, 450, "rcm", 64)])
 @pytest.mark.parametrize("kw", [dict(), dict(soa=True), dict(mixed=True)],
                          ids=["fp64", "soa", "mixed"])
 def test_half_steps_equal_unfused_loops(I, J, ordering, block, kw):
+    """640x450 in patches of 64: more of them than one launch has workgroups
+    (at most 4096), so each walks two.  1024 cells and the rows around them do
+    not fit in 64 KiB and run unfused."""
     mesh = op2amd.mesh.generate(I, J, 3, ordering)
-    fused, plain = fused_and_not(mesh, 29, block_res=block, **kw)
+    fused, plain, halves = fused_and_not(mesh, 29, block_res=block, **kw)
+    assert fused["graph_steps"] == 4 and halves == (0 if block == 1024 else 8)
     for k in KEYS:
         assert np.array_equal(fused[k], plain[k]), k
     if not kw:
@@ -49,24 +59,26 @@ def test_wide_patches_run_unfused(renumber):
     """75,000 randomly numbered cells: a patch's cells span more than 16 bits
     unless the device renumbers them."""
     mesh = op2amd.mesh.generate(300, 250, 5, "random")
-    fused, plain = fused_and_not(mesh, 13, block_res=128, renumber=renumber)
+    fused, plain, halves = fused_and_not(mesh, 13, block_res=128, renumber=renumber)
+    assert fused["graph_steps"] == 4 and halves == (8 if renumber else 0)
     for k in KEYS:
         assert np.array_equal(fused[k], plain[k]), k
 
 
 STEP = ["save_soln"] + 2 * ["adt_calc", "res_calc", "bres_calc", "update"]
+# the captured loops, and how many half steps they hold
 SEQUENCES = {
-    "step": STEP,
-    "three steps": 3 * STEP,
-    "step, then one stage": STEP + ["save_soln", "adt_calc", "res_calc", "bres_calc", "update"],
-    "one stage, twice": 2 * ["save_soln", "adt_calc", "res_calc", "bres_calc", "update"],
-    "ends on save_soln": STEP + ["save_soln"],
-    "ends on adt_calc": 2 * STEP + ["save_soln", "adt_calc"],
-    "ends on res_calc": STEP + ["save_soln", "adt_calc", "res_calc"],
-    "ends on bres_calc": STEP + STEP[:-1],
-    "starts inside a step": STEP[1:] + STEP,
-    "no save_soln": STEP[1:] + STEP[1:],
-    "a second adt_calc": STEP[:2] + ["adt_calc"] + STEP[2:] + STEP,
+    "step": (STEP, 2),
+    "three steps": (3 * STEP, 6),
+    "step, then one stage": (STEP + ["save_soln", "adt_calc", "res_calc", "bres_calc", "update"], 2),
+    "one stage, twice": (2 * ["save_soln", "adt_calc", "res_calc", "bres_calc", "update"], 0),
+    "ends on save_soln": (STEP + ["save_soln"], 2),
+    "ends on adt_calc": (2 * STEP + ["save_soln", "adt_calc"], 4),
+    "ends on res_calc": (STEP + ["save_soln", "adt_calc", "res_calc"], 2),
+    "ends on bres_calc": (STEP + STEP[:-1], 2),
+    "starts inside a step": (STEP[1:] + STEP, 2),
+    "no save_soln": (STEP[1:] + STEP[1:], 0),
+    "a second adt_calc": (STEP[:2] + ["adt_calc"] + STEP[2:] + STEP, 2),
 }
 
 
@@ -96,6 +108,7 @@ def test_captured_sequences_leave_every_dat_as_eager_loops_do(name, soa):
     qold, adt and res, against the same loops run eagerly."""
     mesh = op2amd.mesh.generate(70, 41, 2, "rcm")
     q, res = inputs(mesh, 4)
+    loops, halves = SEQUENCES[name]
 
     def run(captured):
         app = Program(mesh, q, res, soa=soa)
@@ -106,15 +119,17 @@ def test_captured_sequences_leave_every_dat_as_eager_loops_do(name, soa):
             app.play(STEP)  # builds the plans
             out = []
             if captured:
+                n0 = api.op2h_half_step_count()
                 assert api.lib.op2h_graph_begin() == 0
-                app.play(SEQUENCES[name])
+                app.play(loops)
                 assert api.lib.op2h_graph_end() == 0
+                assert api.op2h_half_step_count() - n0 == halves
             for _ in range(3):
                 if captured:
                     assert api.lib.op2h_graph_launch(1) == 0
                     api.op2h_device_sync()
                 else:
-                    app.play(SEQUENCES[name])
+                    app.play(loops)
                 out.append(app.state())
             return out
         finally:
@@ -148,9 +163,11 @@ def test_steps_on_another_res_read_and_zero_it(names):
             for app.res in (second, first):  # builds the plans; both hold values again
                 app.play(STEP[:-1])
             if captured:
+                n0 = api.op2h_half_step_count()
                 assert api.lib.op2h_graph_begin() == 0
                 play()
                 assert api.lib.op2h_graph_end() == 0
+                assert api.op2h_half_step_count() - n0 == (4 if names == "two steps" else 2)
                 assert api.lib.op2h_graph_launch(1) == 0
                 api.op2h_device_sync()
             else:
@@ -181,16 +198,18 @@ def test_equal_maxima_keep_the_lowest_application_index(names):
     for first in (0, 1, 2, 3, 5, 8, 20):
         res = np.zeros((mesh.ncell, 4))
         res[first:, 0] = 2.0 ** -10
-        app = Program(mesh, q, res, tokens=("OP_HIP_RENUMBER",))
+        app = Program(mesh, q, res, tokens=("OP_HIP_RENUMBER=pecell",))
         try:
             api.op2h_set_sync_mode(api.SYNC_GBL_ONLY)
             api.op2h_set_loop_plan(b"res_calc", api.PLAN_OWNER, 64)
             api.op2h_set_loop_plan(b"bres_calc", api.PLAN_GATHER, 128)
             app.play(["adt_calc", "res_calc", "bres_calc"])  # builds the plans
             if captured:
+                n0 = api.op2h_half_step_count()
                 assert api.lib.op2h_graph_begin() == 0
                 app.play(names)
                 assert api.lib.op2h_graph_end() == 0
+                assert api.op2h_half_step_count() - n0 == (2 if names == STEP else 0)
                 assert api.lib.op2h_graph_launch(1) == 0
                 record, n = np.zeros(6), C.c_int()
                 api.lib.op2h_graph_history(1, record.ctypes.data_as(C.c_void_p), C.byref(n))
