@@ -1670,7 +1670,8 @@ void make_half_mem() {
             return op2h_plan_user(name, bytes, &fresh);
           },
           &M.patches, &M.nc, &M.nn) ||
-      patch_lds_bytes<double>(M.nc, M.nn) > 64 * 1024)
+      (R.mixed ? patch_lds_bytes<float>(M.nc, M.nn) : patch_lds_bytes<double>(M.nc, M.nn)) >
+          kPatchLds)
     return;
   const size_t rows = (size_t)(R.soa ? R.cells->stride : R.cells->size);
   const size_t b_q = 4 * sizeof(double) * rows;

@@ -633,7 +633,7 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
                             [&](size_t bytes) { return dev_alloc<char>(bytes, keep); }, &PA,
                             &pa_nc, &pa_nn);
   const size_t half_lds = patch_lds_bytes<double>(pa_nc, pa_nn);
-  half = half && half_lds <= 64 * 1024;
+  half = half && half_lds <= kPatchLds;
   // whole waves: the reductions shuffle over 64 lanes, and the lanes past a
   // patch's cells hold nothing
   const int half_blk = (patch + 63) / 64 * 64;

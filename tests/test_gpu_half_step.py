@@ -42,11 +42,11 @@ def fused_and_not(mesh, niter, **kw):
                          ids=["fp64", "soa", "mixed"])
 def test_half_steps_equal_unfused_loops(I, J, ordering, block, kw):
     """640x450 in patches of 64: more of them than one launch has workgroups
-    (at most 4096), so each walks two.  1024 cells and the rows around them do
-    not fit in 64 KiB and run unfused."""
+    (at most 4096), so each walks two.  Of 1024 cells and the rows around them
+    one patch at a time fits in the LDS of a CU."""
     mesh = op2amd.mesh.generate(I, J, 3, ordering)
     fused, plain, halves = fused_and_not(mesh, 29, block_res=block, **kw)
-    assert fused["graph_steps"] == 4 and halves == (0 if block == 1024 else 8)
+    assert fused["graph_steps"] == 4 and halves == 8
     for k in KEYS:
         assert np.array_equal(fused[k], plain[k]), k
     if not kw:
