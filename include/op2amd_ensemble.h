@@ -119,6 +119,10 @@ int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
                         const op2amd_ensemble_opts *opts,
                         op2amd_ensemble_result *res);
 
+/* Half steps launched as one kernel each (eagerly, or into a graph) since the
+ * library loaded: none where the loops of a run have launches of their own. */
+unsigned long long op2amd_ensemble_half_steps(void);
+
 #ifdef __cplusplus
 }
 #endif

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <chrono>
 #include <cmath>
@@ -336,6 +337,12 @@ template <class T> T *dev_alloc(size_t n, std::vector<void *> &keep) {
 }
 
 }  // namespace
+
+namespace {
+std::atomic<unsigned long long> g_half_steps{0};
+}
+
+extern "C" unsigned long long op2amd_ensemble_half_steps(void) { return g_half_steps; }
 
 extern "C" int op2amd_ensemble_describe(const op2amd_ensemble_spec *spec,
                                         op2amd_ensemble_member *members) {
@@ -757,9 +764,11 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
       // every workgroup walks the same number of patches, give or take one
       const int most = std::max(1, std::min(p1 - p0, cap[3 * k]));
       const int rounds = (p1 - p0 + most - 1) / most, grid = (p1 - p0 + rounds - 1) / std::max(1, rounds);
-      if (p1 > p0)
+      if (p1 > p0) {
         (k ? k_ens_half<true> : k_ens_half<false>)<<<grid, half_blk, half_lds, st>>>(
             H, PA, BA, d_pmember, pa_nc, pa_nn, p0, p1, parts, S_at(off_res[k]));
+        ++g_half_steps;
+      }
     }
     for (int k = 0; k < 2 && !half; ++k) {
       mark();

@@ -44,6 +44,9 @@ lib.op2amd_ensemble_describe.restype = C.c_int
 lib.op2amd_ensemble_describe.argtypes = [C.POINTER(Spec), C.POINTER(Member)]
 lib.op2amd_ensemble_run.restype = C.c_int
 lib.op2amd_ensemble_run.argtypes = [C.POINTER(Spec), C.POINTER(Opts), C.POINTER(Result)]
+lib.op2amd_ensemble_half_steps.restype = C.c_ulonglong
+lib.op2amd_ensemble_half_steps.argtypes = []
+half_steps = lib.op2amd_ensemble_half_steps
 
 
 def spec(nmesh=256, min_IJ=(40, 20), max_IJ=(640, 320), seed=0, mach=(0.3, 0.6),

@@ -28,14 +28,17 @@ def test_members_deterministic_and_in_range():
 def test_batched_equals_looped_and_each_member_equals_sequential_run(ordering):
     """Batched (graphed and eager) and looped runs give the same bits, and each
     member equals the oracle's sequential run of that member.  With random
-    member numberings the owner patches span more than 16-bit offsets and
-    read 16-byte instance records; with RCM they fit the 8-byte form."""
+    member numberings the owner patches span more than 16-bit offsets, the
+    loops have launches of their own and read 16-byte instance records; with
+    RCM they run as half steps."""
     # random: two 400x200 members (80,000 cells, spans beyond 65535)
     cfg = SMALL if ordering == "rcm" else dict(nmesh=2, min_IJ=(400, 200), max_IJ=(400, 200),
                                                seed=3, ordering="random")
     sp = op2amd.ensemble.spec(**cfg)
     niter = 60
+    n0 = op2amd.ensemble.half_steps()
     batched = op2amd.ensemble.run(sp, niter, batched=True, graphed=True, want_q=True)
+    assert op2amd.ensemble.half_steps() - n0 == (2 * 10 if ordering == "rcm" else 0)
     eager = op2amd.ensemble.run(sp, niter, batched=True, graphed=False, want_q=True)
     looped = op2amd.ensemble.run(sp, niter, batched=False, want_q=True)
     for r in (eager, looped):
@@ -55,20 +58,28 @@ def test_batched_equals_looped_and_each_member_equals_sequential_run(ordering):
 
 
 @pytest.mark.gpu
-def test_autotuned_block_sizes_change_no_bits():
+@pytest.mark.parametrize("form", ["half steps", "bres_calc apart", "wide patches"])
+def test_autotuned_block_sizes_change_no_bits(form):
     """The batched run with its workgroup sizes picked by timing the first
     ten steps (one candidate per step, each twice) gives the bits of the default launch
-    shapes; the picks are candidates."""
-    sp = op2amd.ensemble.spec(**SMALL)
-    plain = op2amd.ensemble.run(sp, 30, batched=True, graphed=True, want_q=True)
-    tuned = op2amd.ensemble.run(sp, 30, batched=True, graphed=True, want_q=True,
-                                autotune=True)
+    shapes; the picks are candidates.  Half steps have nothing to pick; with
+    bres_calc apart, and where patches span more than 16 bits (randomly
+    numbered members of 80,000 cells), the loops run in launches of their own."""
+    sp = op2amd.ensemble.spec(**(SMALL if form != "wide patches" else dict(
+        nmesh=2, min_IJ=(400, 200), max_IJ=(400, 200), seed=3, ordering="random")))
+    kw = dict(batched=True, graphed=True, want_q=True, separate_bres=form == "bres_calc apart")
+    n0 = op2amd.ensemble.half_steps()
+    plain = op2amd.ensemble.run(sp, 30, **kw)
+    tuned = op2amd.ensemble.run(sp, 30, autotune=True, **kw)
+    # 30 steps from one captured graph of ten, in either run
+    assert op2amd.ensemble.half_steps() - n0 == (2 * 2 * 10 if form == "half steps" else 0)
     for key in ("rms", "maxerr", "errloc", "q"):
         assert np.array_equal(tuned[key], plain[key]), key
-    # bres_calc runs inside res_calc's launch: no workgroup size of its own
-    assert plain["blocks"] == {"update_adt": 256, "res_calc": 256, "bres_calc": 0,
+    # bres_calc runs inside res_calc's launch unless apart: no workgroup size of its own
+    apart = form == "bres_calc apart"
+    assert plain["blocks"] == {"update_adt": 256, "res_calc": 256, "bres_calc": 128 if apart else 0,
                                "update_save_adt": 256}
-    assert plain["fused_bres"] and tuned["fused_bres"]
+    assert plain["fused_bres"] == tuned["fused_bres"] == (not apart)
     assert set(tuned["blocks"].values()) <= {0, 64, 128, 256, 512, 1024}
     assert tuned["blocks"]["res_calc"] == 256
     assert plain["dead_res"] and tuned["dead_res"]
