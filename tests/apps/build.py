@@ -48,6 +48,10 @@ FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
+def reference_present():
+    return os.path.isdir(os.path.join(REFERENCE, "apps"))
+
+
 def build(name):
     from op2amd.translator import translate
     if name in REF_PROGRAMS:
@@ -75,6 +79,6 @@ def build(name):
 
 
 if __name__ == "__main__":
-    names = sys.argv[1:] or [*PROGRAMS, *(REF_PROGRAMS if os.path.isdir(os.path.join(REFERENCE, "apps")) else [])]
+    names = sys.argv[1:] or [*PROGRAMS, *(REF_PROGRAMS if reference_present() else [])]
     for n in names:
         print(build(n), flush=True)

@@ -1,3 +1,4 @@
+import importlib.util
 import pathlib
 import sys
 
@@ -34,6 +35,22 @@ def pointwise_rel_err(a, b):
     d = np.abs(a - b)
     s = np.abs(b)
     return float(np.max(np.where(s > 0, d / np.where(s > 0, s, 1.0), d)))
+
+
+def _apps():
+    spec = importlib.util.spec_from_file_location("apps_build", REPO / "tests" / "apps" / "build.py")
+    m = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(m)
+    return m
+
+
+def reference_program(path):
+    """A program that __graft_entry__.build() builds from the reference's own
+    sources: the test is skipped only where those are absent too."""
+    if not path.exists():
+        assert not _apps().reference_present(), f"{path} missing: run __graft_entry__.build()"
+        pytest.skip(f"{path} missing, and so are the sources it is built from")
+    return path
 
 
 @pytest.fixture(scope="session")

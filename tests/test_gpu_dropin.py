@@ -31,7 +31,7 @@ import numpy as np
 import pytest
 
 import op2amd
-from conftest import REPO, golden
+from conftest import REPO, golden, reference_program
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -39,8 +39,7 @@ EXE = REPO / "tests" / "apps" / "_build" / "airfoil_ref" / "airfoil_ref"
 
 
 def run_app(tmp_path, *tokens, env_extra=None):
-    if not EXE.exists():  # built from the reference's sources only
-        pytest.skip(f"{EXE} missing: run __graft_entry__.build() where the reference is present")
+    reference_program(EXE)
     g = golden("airfoil_24x12_random_app_a0")
     mesh = op2amd.mesh.generate(int(g["I"]), int(g["J"]), 0, str(g["ordering"]))
     mesh.write(str(tmp_path / "new_grid.dat"))
@@ -55,9 +54,7 @@ def run_app(tmp_path, *tokens, env_extra=None):
 
 def run_variant(tmp_path, exe, golden_name, *tokens):
     """A reference app variant on its golden's mesh; its printed history."""
-    path = REPO / "tests" / "apps" / "_build" / exe / exe
-    if not path.exists():
-        pytest.skip(f"{path} missing: run __graft_entry__.build() where the reference is present")
+    path = reference_program(REPO / "tests" / "apps" / "_build" / exe / exe)
     g = golden(golden_name)
     mesh = op2amd.mesh.generate(int(g["I"]), int(g["J"]), 0, str(g["ordering"]))
     mesh.write(str(tmp_path / "new_grid.dat"))

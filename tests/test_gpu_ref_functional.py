@@ -9,7 +9,7 @@ also checked on the host.  Run with the default plans, every dat in SoA
 layout, coloured and atomic increments, and under transparent renumbering."""
 import pytest
 
-from conftest import REPO
+from conftest import REPO, reference_program
 
 pytestmark = pytest.mark.gpu
 BUILD = REPO / "tests" / "apps" / "_build"
@@ -24,9 +24,7 @@ CHECKS = {"ref_gbl": 8, "ref_reduc": 4, "ref_idx": 3, "ref_strides": 2, "ref_con
 @pytest.mark.parametrize("name", sorted(CHECKS))
 def test_reference_functional_test(name, variant, tmp_path):
     import subprocess
-    exe = BUILD / name / name
-    if not exe.exists():  # built from the reference's sources only
-        pytest.skip(f"{exe} missing: run __graft_entry__.build() where the reference is present")
+    exe = reference_program(BUILD / name / name)
     print("running", name, *variant, flush=True)
     r = subprocess.run([str(exe), *variant], cwd=tmp_path, capture_output=True, text=True,
                        timeout=120)
