@@ -332,6 +332,15 @@ const op2h_color_plan *op2h_plan_color_for(const char *name, op_set set,
  * any graph capture). */
 void *op2h_plan_user(const char *key, size_t bytes, int *fresh);
 
+/* Device memory that only makes things faster: NULL, with no error left
+ * behind, where the device has no room for it (hipFree gives it back), and the
+ * caller takes the way that needs none.  op2h_extra_plan_user: the same for a
+ * buffer as of op2h_plan_user.  op2h_set_extra_memory: nothing above `bytes` at
+ * a time is asked for (default: no such limit; kept across op_init/op_exit). */
+void *op2h_extra_alloc(size_t bytes);
+void *op2h_extra_plan_user(const char *key, size_t bytes, int *fresh);
+void op2h_set_extra_memory(size_t bytes);
+
 /* Under transparent renumbering (op_init token OP_HIP_RENUMBER or
  * OP_HIP_RENUMBER=<map>): before the first loop the runtime renumbers the
  * sets as op_renumber(<map>) would (default map: the first declared one of

@@ -1519,7 +1519,8 @@ void flush_halves(void *) { launch_recorded(false, false, false); }
 // map (bedge -> cell), built on the device once per plan: each owned cell's
 // interior increments, then its boundary edges (ascending; under transparent
 // renumbering in the application's order).  Null when a cell has more than
-// four increments in all, or the local ids do not fit 15 bits.
+// four increments in all, the local ids do not fit 15 bits, or the device has
+// no room to build them.
 struct BoundaryRec {
   unsigned epoch = 0;  // op2h_plan_epoch() when built
   bool ok = false;
@@ -1556,8 +1557,8 @@ const BoundaryArgs *boundary_args(const op2h_owner_plan *p, op_map pbecell, op_m
   // scratch: each owned cell's boundary edges and their number, each cell's
   // position, each block's number, the flag
   const size_t b_slots = (size_t)16 * no, b_cnt = (size_t)4 * no, b_pos = (size_t)4 * ncell;
-  char *tmp = nullptr;
-  KCHECK(hipMalloc(&tmp, b_slots + b_cnt + b_pos + 4 * (size_t)nb + 4));
+  char *tmp = (char *)op2h_extra_alloc(b_slots + b_cnt + b_pos + 4 * (size_t)nb + 4);
+  if (!tmp) return nullptr;
   int4 *slots = (int4 *)tmp;
   int *cnt = (int *)(tmp + b_slots), *pos = (int *)(tmp + b_slots + b_cnt);
   int *total = (int *)(tmp + b_slots + b_cnt + b_pos), *bad = total + nb;
@@ -1648,7 +1649,8 @@ void pack_compact_rows(op_map m, hipStream_t st) {
 }
 
 // The memory of the fused half steps, for the latest owner-plan res_calc and
-// the latest adt_calc's map when they are over the same cells.
+// the latest adt_calc's map when they are over the same cells, and the device
+// has room (62 bytes a cell or so).
 void make_half_mem() {
   const PendingRes &R = g_last_res;
   const op_map pcell = g_last_pcell.map;
@@ -1667,7 +1669,7 @@ void make_half_mem() {
           R.A, p->nblocks, g_last_bres.rec, (const int4 *)pcell->map_d, R.cells->size, R.st,
           [&](size_t bytes) {
             snprintf(name, sizeof name, "half_step.lists%d.%p", part++, (const void *)p);
-            return op2h_plan_user(name, bytes, &fresh);
+            return op2h_extra_plan_user(name, bytes, &fresh);
           },
           &M.patches, &M.nc, &M.nn) ||
       (R.mixed ? patch_lds_bytes<float>(M.nc, M.nn) : patch_lds_bytes<double>(M.nc, M.nn)) >
@@ -1676,8 +1678,9 @@ void make_half_mem() {
   const size_t rows = (size_t)(R.soa ? R.cells->stride : R.cells->size);
   const size_t b_q = 4 * sizeof(double) * rows;
   snprintf(name, sizeof name, "half_step.q.%p", (const void *)p);
-  M.q2 = (double *)op2h_plan_user(
+  M.q2 = (double *)op2h_extra_plan_user(
       name, b_q + (R.mixed ? sizeof(float) : sizeof(double)) * rows, &fresh);
+  if (!M.q2) return;
   M.adt2 = (char *)M.q2 + b_q;
   M.epoch = now;
   M.plan = p;

@@ -427,9 +427,9 @@ static __global__ void __launch_bounds__(256)
 }
 
 // Builds the lists for an owner partition whose every cell (ncell of them) is
-// owned; `alloc(bytes)` gives device memory that outlives them.  Returns false
-// when a patch does not fit (any memory asked for then is unused).  Blocks
-// until the device has built them.
+// owned; `alloc(bytes)` gives device memory that outlives them, or null.
+// Returns false when a patch does not fit or there is no memory (any asked for
+// then is unused).  Blocks until the device has built them.
 template <class Alloc>
 bool build_patches(const OwnerArgs &O, int nblocks, const ushort4 *rec, const int4 *pcell,
                    int ncell, hipStream_t st, Alloc alloc, PatchArgs *out, int *nc_max,
@@ -442,6 +442,7 @@ bool build_patches(const OwnerArgs &O, int nblocks, const ushort4 *rec, const in
   };
   const size_t b_info = 256, b_pos = ((size_t)4 * ncell + 255) / 256 * 256;
   char *mem = (char *)alloc(b_info + b_pos);
+  if (!mem) return false;
   int *info = (int *)mem, *pos = (int *)(mem + b_info);
   const int zeros[3] = {0, 0, 0};
   int got[3];
@@ -458,6 +459,7 @@ bool build_patches(const OwnerArgs &O, int nblocks, const ushort4 *rec, const in
   const size_t b_ent = ((size_t)8 * ncell + 255) / 256 * 256;
   const size_t b_cells = ((size_t)2 * cs * nblocks + 255) / 256 * 256;
   char *m = (char *)alloc(b_head + 2 * b_ent + b_cells + (size_t)2 * ns * nblocks);
+  if (!m) return false;
   int4 *head = (int4 *)m;
   uint2 *edges = (uint2 *)(m + b_head), *corners = (uint2 *)(m + b_head + b_ent);
   unsigned short *cells = (unsigned short *)(m + b_head + 2 * b_ent);

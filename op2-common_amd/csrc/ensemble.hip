@@ -327,6 +327,16 @@ template <class T> T *dev_upload(const std::vector<T> &v, std::vector<void *> &k
   return (T *)p;
 }
 
+// Zeroed like dev_alloc's, or null where the device has no room.
+void *dev_try(size_t bytes, std::vector<void *> &keep) {
+  void *p = op2h_extra_alloc(std::max<size_t>(bytes, 1));
+  if (!p) return nullptr;
+  ECHECK(hipMemset(p, 0, std::max<size_t>(bytes, 1)));
+  ECHECK(hipDeviceSynchronize());
+  keep.push_back(p);
+  return p;
+}
+
 template <class T> T *dev_alloc(size_t n, std::vector<void *> &keep) {
   void *p = nullptr;
   ECHECK(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)));
@@ -628,24 +638,25 @@ extern "C" int op2amd_ensemble_run(const op2amd_ensemble_spec *spec,
   int2 *d_tiles = dev_upload(tiles, keep);
   int *d_coff = dev_upload(coff, keep);
   int *d_mtoff = dev_upload(mesh_tile_off, keep);
-  // the half steps' memory: where bres_calc is not kept apart and every patch
-  // fits its lists, each half step is one launch (k_ens_half); else the chains
-  // and res_calc + bres_calc
+  // the half steps' memory: where bres_calc is not kept apart, every patch fits
+  // its lists and the device has room, each half step is one launch
+  // (k_ens_half); else the chains and res_calc + bres_calc
   hipStream_t st;
   ECHECK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
   PatchArgs PA{};
   int pa_nc = 0, pa_nn = 0;
   bool half = fused && npatch > 0 &&
               build_patches(OA, npatch, BA.rec, d_cell, Nc, st,
-                            [&](size_t bytes) { return dev_alloc<char>(bytes, keep); }, &PA,
+                            [&](size_t bytes) { return dev_try(bytes, keep); }, &PA,
                             &pa_nc, &pa_nn);
   const size_t half_lds = patch_lds_bytes<double>(pa_nc, pa_nn);
   half = half && half_lds <= kPatchLds;
   // whole waves: the reductions shuffle over 64 lanes, and the lanes past a
   // patch's cells hold nothing
   const int half_blk = (patch + 63) / 64 * 64;
-  double *d_q2 = half ? dev_alloc<double>(4 * (size_t)Nc, keep) : nullptr;
-  double *d_adt2 = half ? dev_alloc<double>(Nc, keep) : nullptr;
+  double *d_q2 = half ? (double *)dev_try(5 * sizeof(double) * (size_t)Nc, keep) : nullptr;
+  half = half && d_q2;
+  double *d_adt2 = half ? d_q2 + 4 * (size_t)Nc : nullptr;
   std::vector<int2> pmember(npatch);
   for (int m = 0; m < M; ++m)
     for (int b = mblk[m]; b < mblk[m + 1]; ++b) pmember[b] = make_int2(m, coff[m]);

@@ -270,13 +270,18 @@ __global__ void k_csr4(const int *__restrict csr_offs, const unsigned short *__r
 
 int grid(size_t n) { return (int)((n + 255) / 256); }
 
-// Device scratch of one build, freed at its end.
+// Device scratch of one build, freed at its end.  full: the device had no room
+// for some of it (null), and the host builds the plan.
 struct Scratch {
   std::vector<void *> ptrs;
+  bool full = false;
   template <class T> T *get(size_t n, bool zero, hipStream_t st) {
-    void *p = nullptr;
     const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 3) / 4 * 4;
-    OGCHECK(hipMalloc(&p, bytes));
+    void *p = full ? nullptr : op2h_extra_alloc(bytes);
+    if (!p) {
+      full = true;
+      return nullptr;
+    }
     if (zero) OGCHECK(hipMemsetAsync(p, 0, bytes, st));
     ptrs.push_back(p);
     return (T *)p;
@@ -304,6 +309,7 @@ bool gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc, con
   const Map m = map_of(nto, nel, dim, map_d, ninc, inc_idx);
   int *deg = S.get<int>((size_t)nto + 1, true, st), *width = S.get<int>(1, true, st);
   unsigned char *used = S.get<unsigned char>(nto, true, st);
+  if (S.full) return false;
   k_degrees<<<grid(nel), 256, 0, st>>>(m, deg, used, width);
   g.off.resize((size_t)nto + 1);
   g.used.resize(nto);
@@ -324,6 +330,7 @@ bool gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc, con
   if (!n) return true;
   int *off = S.get<int>((size_t)nto + 1, false, st), *out = S.get<int>(n, false, st);
   unsigned long long *adj = S.get<unsigned long long>(n, false, st);
+  if (S.full) return false;
   OGCHECK(hipMemcpyAsync(off, g.off.data(), sizeof(int) * ((size_t)nto + 1),
                          hipMemcpyHostToDevice, st));
   OGCHECK(hipMemsetAsync(deg, 0, sizeof(int) * nto, st));
@@ -342,6 +349,10 @@ bool gpu_owner_lists(int nto, int nel, int dim, const int *map_d, int ninc, cons
   op2h_owner_plan &P = rec.plan;
   const Map m = map_of(nto, nel, dim, map_d, ninc, inc_idx);
   int *blk = S.get<int>(nto, false, st), *cnt = S.get<int>(3 * (size_t)nb, true, st);
+  int *inc_offs = S.get<int>((size_t)nb + 1, false, st);
+  int *key = elem_key ? S.get<int>(nel, false, st) : nullptr;
+  int *pos = S.get<int>(nto, false, st), *longest = S.get<int>(1, true, st);
+  if (S.full) return false;
   OGCHECK(hipMemcpyAsync(blk, block_of.data(), sizeof(int) * nto, hipMemcpyHostToDevice, st));
   const int g = grid(std::max(nto, nel));
   k_block_counts<<<g, 256, 0, st>>>(m, blk, nb, cnt);
@@ -361,18 +372,12 @@ bool gpu_owner_lists(int nto, int nel, int dim, const int *map_d, int ninc, cons
   if (most[0] > kSortMax || most[1] > kSortMax || (long long)most[1] * ninc > 65535) return false;
   const int n_owned = offs[0][nb], total = offs[1][nb], n_csr = offs[2][nb];
   int *owned_offs = rec.mem.upload(offs[0], st), *elem_offs = rec.mem.upload(offs[1], st);
-  int *inc_offs = S.get<int>((size_t)nb + 1, false, st);
   OGCHECK(hipMemcpyAsync(inc_offs, offs[2].data(), sizeof(int) * ((size_t)nb + 1),
                          hipMemcpyHostToDevice, st));
-  int *key = nullptr;
-  if (elem_key) {
-    key = S.get<int>(nel, false, st);
-    OGCHECK(hipMemcpyAsync(key, elem_key, sizeof(int) * nel, hipMemcpyHostToDevice, st));
-  }
+  if (key) OGCHECK(hipMemcpyAsync(key, elem_key, sizeof(int) * nel, hipMemcpyHostToDevice, st));
   int *owned = rec.mem.alloc<int>(n_owned), *elems = rec.mem.alloc<int>(total);
   int *csr_offs = rec.mem.alloc<int>((size_t)n_owned + 1);
   unsigned short *csr = rec.mem.alloc<unsigned short>(n_csr);
-  int *pos = S.get<int>(nto, false, st), *longest = S.get<int>(1, true, st);
   OGCHECK(hipMemsetAsync(cnt, 0, sizeof(int) * 2 * (size_t)nb, st));
   k_block_fill<<<g, 256, 0, st>>>(m, blk, nb, owned_offs, elem_offs, cnt, owned, elems);
   k_block_order<<<nb, 256, 0, st>>>(owned_offs, owned, elem_offs, elems,

@@ -125,7 +125,8 @@ struct TargetGraph {
 // table: the graph (false, and the graph unset, when a target has more
 // neighbours than a list could hold), and a plan's lists for patches grown over
 // it (false, and the record's lists unset, when a block or a target's list is
-// too long for it); both block until built.  gpu_owner_fits: whether the loop's
+// too long for it); both false too where the device has no room for their
+// scratch, and blocking until built.  gpu_owner_fits: whether the loop's
 // shape is theirs.
 bool gpu_owner_fits(int nto, int nel, int ninc);
 bool gpu_target_graph(int nto, int nel, int dim, const int *map_d, int ninc,

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -2300,7 +2301,11 @@ extern "C" int op2h_owner_plan_download(const op2h_owner_plan *p,
   return 1;
 }
 
-extern "C" void *op2h_plan_user(const char *key, size_t bytes, int *fresh) {
+namespace {
+std::atomic<size_t> g_extra_memory{SIZE_MAX};
+
+// must: the program ends where the device has no room, else null.
+void *plan_user(const char *key, size_t bytes, int *fresh, bool must) {
   Runtime &R = rt();
   auto it = R.user_plans.find(key);
   if (it != R.user_plans.end() && it->second.second == bytes) {
@@ -2317,10 +2322,31 @@ extern "C" void *op2h_plan_user(const char *key, size_t bytes, int *fresh) {
     R.user_plans.erase(it);
   }
   void *p = nullptr;
-  HIPCHECK(hipMalloc(&p, std::max(bytes, (size_t)16)));
+  const size_t need = std::max(bytes, (size_t)16);
+  if (must) HIPCHECK(hipMalloc(&p, need));
+  else if (!(p = op2h_extra_alloc(need))) return nullptr;
   R.user_plans[key] = {p, bytes};
   *fresh = 1;
   return p;
+}
+}  // namespace
+
+extern "C" void op2h_set_extra_memory(size_t bytes) { g_extra_memory = bytes; }
+
+extern "C" void *op2h_extra_alloc(size_t bytes) {
+  void *p = nullptr;
+  if (bytes > g_extra_memory) return nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+extern "C" void *op2h_plan_user(const char *key, size_t bytes, int *fresh) {
+  return plan_user(key, bytes, fresh, true);
+}
+
+extern "C" void *op2h_extra_plan_user(const char *key, size_t bytes, int *fresh) {
+  return plan_user(key, bytes, fresh, false);
 }
 
 extern "C" int op2h_staged_plan_download(const op2h_staged_plan *p, int *thrcol,

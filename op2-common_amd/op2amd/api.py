@@ -208,6 +208,7 @@ op2h_set_old_index = _fn("op2h_set_old_index", C.c_void_p, op_set)
 op2h_set_fusion = _fn("op2h_set_fusion", None, C.c_int)
 op2h_fused_count = _fn("op2h_fused_count", C.c_ulonglong)
 op2h_half_step_count = _fn("op2h_half_step_count", C.c_ulonglong)
+op2h_set_extra_memory = _fn("op2h_set_extra_memory", None, C.c_size_t)
 op2h_set_streaming = _fn("op2h_set_streaming", None, C.c_int)
 op2h_streaming = _fn("op2h_streaming", C.c_int, C.c_size_t)
 

@@ -58,19 +58,25 @@ def test_batched_equals_looped_and_each_member_equals_sequential_run(ordering):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("form", ["half steps", "bres_calc apart", "wide patches"])
+@pytest.mark.parametrize("form", ["half steps", "bres_calc apart", "wide patches", "no room"])
 def test_autotuned_block_sizes_change_no_bits(form):
     """The batched run with its workgroup sizes picked by timing the first
     ten steps (one candidate per step, each twice) gives the bits of the default launch
     shapes; the picks are candidates.  Half steps have nothing to pick; with
-    bres_calc apart, and where patches span more than 16 bits (randomly
-    numbered members of 80,000 cells), the loops run in launches of their own."""
+    bres_calc apart, where patches span more than 16 bits (randomly numbered
+    members of 80,000 cells), and where the device has no room for the other
+    copies of q and adt, the loops run in launches of their own."""
     sp = op2amd.ensemble.spec(**(SMALL if form != "wide patches" else dict(
         nmesh=2, min_IJ=(400, 200), max_IJ=(400, 200), seed=3, ordering="random")))
     kw = dict(batched=True, graphed=True, want_q=True, separate_bres=form == "bres_calc apart")
     n0 = op2amd.ensemble.half_steps()
-    plain = op2amd.ensemble.run(sp, 30, **kw)
-    tuned = op2amd.ensemble.run(sp, 30, autotune=True, **kw)
+    if form == "no room":
+        op2amd.api.op2h_set_extra_memory(0)
+    try:
+        plain = op2amd.ensemble.run(sp, 30, **kw)
+        tuned = op2amd.ensemble.run(sp, 30, autotune=True, **kw)
+    finally:
+        op2amd.api.op2h_set_extra_memory(2 ** 64 - 1)
     # 30 steps from one captured graph of ten, in either run
     assert op2amd.ensemble.half_steps() - n0 == (2 * 2 * 10 if form == "half steps" else 0)
     for key in ("rms", "maxerr", "errloc", "q"):

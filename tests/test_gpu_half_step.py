@@ -65,6 +65,23 @@ def test_wide_patches_run_unfused(renumber):
         assert np.array_equal(fused[k], plain[k]), k
 
 
+@pytest.mark.parametrize("limit", [0, 30_000, 100_000])
+def test_without_room_the_loops_run_unfused(limit):
+    """Half steps need memory of their own: none of it is there, too little for
+    the scratch of the boundary records (69 kB), or all but the other copies of
+    q and adt (115 kB)."""
+    mesh = op2amd.mesh.generate(61, 47, 3, "rcm")
+    api.op2h_set_extra_memory(limit)
+    try:
+        fused, plain, halves = fused_and_not(mesh, 29, block_res=128)
+    finally:
+        api.op2h_set_extra_memory(2 ** 64 - 1)
+    assert halves == 0
+    for k in KEYS:
+        assert np.array_equal(fused[k], plain[k]), k
+    assert fused_and_not(mesh, 29, block_res=128)[2] == 8
+
+
 STEP = ["save_soln"] + 2 * ["adt_calc", "res_calc", "bres_calc", "update"]
 # the captured loops, and how many half steps they hold
 SEQUENCES = {

@@ -115,3 +115,35 @@ def test_a_target_that_many_elements_name(hub):
     got = np.full(Star.ncell, -1, np.int32)
     got[ow] = np.repeat(np.arange(nb), np.diff(oo))
     assert p.nblocks == nb and np.array_equal(got, block_of)
+
+
+@pytest.mark.parametrize("limit", [0, 100_000, 400_000, 2 ** 50])
+def test_without_room_for_scratch_the_host_builds_the_lists(limit):
+    """27,000 edges: scratch of at most so many bytes at a time, from none at
+    all to the graph's neighbours (430 kB), and no limit."""
+    mesh = op2amd.mesh.generate(147, 93, 4, "random")
+    want = plan_of(mesh, 128)
+    want = lists(want, mesh.nedge)
+    api.op_exit()
+    api.op2h_set_extra_memory(limit)
+    try:
+        got = lists(plan_of(mesh, 128), mesh.nedge)
+    finally:
+        api.op2h_set_extra_memory(2 ** 64 - 1)
+        api.op_exit()
+    n = want[4][-1]
+    for k, (a, b) in enumerate(zip(want, got)):
+        assert np.array_equal(a[:n], b[:n]) if k == 5 else np.array_equal(a, b)
+
+
+def test_more_than_the_device_holds_is_refused_without_an_error():
+    api.init()
+    try:
+        p = api.lib.op2h_extra_alloc
+        p.restype, p.argtypes = C.c_void_p, [C.c_size_t]
+        assert p(1 << 50) is None
+        cells = api.op_decl_set(1000, b"cells")
+        d = api.decl_dat(cells, 1, "double", np.arange(1000.0), "d")
+        assert np.array_equal(api.fetch(d, (1000,), np.float64), np.arange(1000.0))
+    finally:
+        api.op_exit()
