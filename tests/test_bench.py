@@ -33,6 +33,25 @@ def test_roofline_traffic_from_profiles():
     assert gen and 1.0 <= gen / 109.44e6 <= 1.1
     assert large and 1.0 <= large / 1751.0e6 <= 1.1
     assert b.profiled_traffic("res_calc/owner/128", "no-such-mesh") is None
+    # a half step's patch lists (16 bits a row) are shorter than its maps
+    for block in (128, 256):
+        half = b.profiled_traffic(f"half_step/owner/{block}", "1200x600/rcm")
+        assert half and 0.9 <= half / 115.2e6 <= 1.0
+
+
+def test_roofline_names_the_kernel_of_the_timed_graphs():
+    b = load_bench()
+
+    class Mesh:
+        ncell, nedge, nnode = 720_000, 1_438_200, 721_801
+    assert abs(b.half_step_bytes(Mesh) - 115.2e6) < 1e5
+    head = dict(tuned_plans=dict(plan_res="owner", block_res=128), steps_per_graph_launch=10,
+                half_steps_per_graph_launch=20, per_loop=dict(res_calc=dict(achieved_GBs=4800.0)))
+    half = b.roofline(Mesh, head, 16000.0, "1200x600/rcm")
+    assert half["kernel"] == "half_step (owner, block 128)" and half["traffic"] > 1e8
+    assert abs(half["achieved"] - 115.2e6 * 32000 / 1e9) < 5
+    loops = b.roofline(Mesh, dict(head, half_steps_per_graph_launch=0), 16000.0, "1200x600/rcm")
+    assert loops["kernel"] == "res_calc (owner, block 128)" and loops["achieved"] == 4800.0
 
 
 def test_parity_check_flags_a_wrong_iteration():
