@@ -741,9 +741,10 @@ __global__ void __launch_bounds__(1024)
     for (int d = 0; d < 4; ++d) r[d] = (double)rr[d];
     // op_arg_idx: the application's element index (transparent renumbering)
     const int ci = oldidx ? oldidx[c] : c;
-    MaxLoc ml{-INFINITY, 0x7fffffff};
-    op2_k::update(qo, qn, r, &a, &cs, &ml.v, &ci, &ml.loc);
-    op2h_red::add_cell(acc, cs, ml);
+    double mx = -INFINITY;
+    int at;
+    op2_k::update(qo, qn, r, &a, &cs, &mx, &ci, &at);
+    op2h_red::add_cell(acc, cs, mx, ci);
     st4<SOA>(q, c, s, qn);
     const R z[4] = {0, 0, 0, 0};
     st4r<SOA>(res, c, s, z);
@@ -1016,9 +1017,10 @@ __global__ void __launch_bounds__(1024)
       ld4r<SOA>(res, c, s, rr);
       for (int d = 0; d < 4; ++d) r[d] = (double)rr[d];
       const int ci = oldidx ? oldidx[c] : c;
-      MaxLoc ml{-INFINITY, 0x7fffffff};
-      op2_k::update(qo, qn, r, &a, &cs, &ml.v, &ci, &ml.loc);
-      op2h_red::add_cell(acc, cs, ml);
+      double mx = -INFINITY;
+      int at;
+      op2_k::update(qo, qn, r, &a, &cs, &mx, &ci, &at);
+      op2h_red::add_cell(acc, cs, mx, ci);
       st4<SOA>(q, c, s, qn);
       if (!res_dead) {
         const R z[4] = {0, 0, 0, 0};

@@ -237,9 +237,10 @@ __device__ __forceinline__ void half_step_patch(int b, const HalfArgs<R> &H, con
   const double da = (double)a;
   double cs = 0.0;
   const int idx = H.oldidx ? H.oldidx[c] : c - idx0;
-  op2h_red::MaxLoc ml{-INFINITY, 0x7fffffff};
-  op2_k::update(qo, qn, rd, &da, &cs, &ml.v, &idx, &ml.loc);
-  op2h_red::add_cell(acc, cs, ml);
+  double mx = -INFINITY;
+  int at;
+  op2_k::update(qo, qn, rd, &da, &cs, &mx, &idx, &at);
+  op2h_red::add_cell(acc, cs, mx, idx);
   st4<SOA>(H.q_out, c, H.sq, qn);
   if (H.flags & (kHalfZeroRes | kHalfCopyAdt | kHalfSaveOld | kHalfSaveNew)) {
     const R z[4] = {0, 0, 0, 0};

@@ -137,12 +137,13 @@ struct UpdateAcc {
   MaxLoc ml{-INFINITY, 0x7fffffff};
 };
 
-// One cell's share, its sum and its own maximum: joined as any other maximum,
-// because the cells a thread takes need not come in index order (a thread's
-// running maximum would keep the first it visits of two equal ones).
-__device__ __forceinline__ void add_cell(UpdateAcc &a, double sum, MaxLoc ml) {
+// One cell's share, its sum and its own maximum `mx` (-infinity where it has
+// none, every change being NaN): joined as any other maximum, because the cells
+// a thread takes need not come in index order (a thread's running maximum would
+// keep the first it visits of two equal ones).
+__device__ __forceinline__ void add_cell(UpdateAcc &a, double sum, double mx, int idx) {
   sum2_add(a.rms, sum);
-  a.ml = maxloc_combine(a.ml, ml);
+  a.ml = maxloc_combine(a.ml, MaxLoc{mx, mx > -INFINITY ? idx : 0x7fffffff});
 }
 
 __device__ __forceinline__ void wave_join(UpdateAcc &a) {
