@@ -3,19 +3,19 @@
  *
  * An ensemble is many airfoil problems of different sizes and free streams
  * advanced in lock step.  All member meshes are concatenated into one set of
- * nodes/cells/edges/bedges; each loop's work is a table of items, runs of one
- * member's elements (tiles of <= 1024 cells, the owner patches of res_calc
- * with bres_calc inside them, or <= 64 boundary cells when bres_calc runs
- * apart), with per-member offsets into it.  Each
- * loop of the time step is ONE persistent launch over every member's items: a
- * grid of as many workgroups as the GPU holds at once, each walking the item
- * table (no edge crosses members, so the concatenation is exact).  update,
- * save_soln and adt_calc of a cell run in one pass (the update of the second
- * half step does the next step's save_soln and adt_calc; one save_soln and
- * adt_calc launch precedes the first step), the per-member rms/maxerr/errloc
- * reductions run through per-tile partials, and the whole time step is
- * captured in one HIP graph.  The baseline launches every loop once per
- * member.  The arithmetic per element is the single-mesh airfoil's
+ * nodes/cells/edges/bedges (no edge crosses members, so the concatenation is
+ * exact).  A half step, res_calc, bres_calc, update and the save_soln and
+ * adt_calc that follow, is ONE persistent launch over every member's owner
+ * patches: a grid of as many workgroups as the GPU holds at once, each walking
+ * the patches.  Where bres_calc is kept apart, a patch does not fit its 16-bit
+ * lists or the LDS, or the device has no room for the other copies of q and
+ * adt, each loop is a persistent launch of its own over a table of items, runs
+ * of one member's elements (tiles of <= 1024 cells for update, save_soln and
+ * adt_calc in one pass, the owner patches of res_calc, <= 64 boundary cells of
+ * bres_calc).  One save_soln and adt_calc launch precedes the first step, the
+ * per-member rms/maxerr/errloc reductions run through partials of one member's
+ * cells each, and ten time steps are captured in one HIP graph.  The baseline
+ * launches the same once per member.  The arithmetic per element is the single-mesh airfoil's
  * (owner-compute res_calc/bres_calc), so each member's trajectory equals its
  * own sequential run (airfoil.cpp:221-297) bit for bit in q.
  *
@@ -60,7 +60,7 @@ int op2amd_ensemble_describe(const op2amd_ensemble_spec *spec,
 typedef struct {
   int niter, warmup;
   int batched;     /* 1: one launch per loop for all members; 0: per member */
-  int graphed;     /* batched only: time step replayed from a HIP graph */
+  int graphed;     /* batched only: time steps replayed from HIP graphs */
   int member_timing; /* per-member step times: looped mode, HIP events around
                         each member's launches; batched mode, device-clock
                         stamps of every work item inside the batched step
@@ -104,7 +104,9 @@ typedef struct {
   int blocks[4];        /* workgroup sizes: update+adt_calc (first half
                            step), res_calc (its owner patch size), bres_calc
                            (0: fused into res_calc), update+save_soln+adt_calc
-                           (second half step) */
+                           (second half step); where half steps are launches
+                           of their own, theirs (the patch size rounded up to
+                           a multiple of 64) in the first and the last */
   int grids[4];         /* persistent grids (workgroups) of the same launches
                            over all members */
   int dead_res;         /* 1: every cell is owned by a res_calc patch, so the

@@ -990,7 +990,7 @@ namespace {
 
 // R: the type of res and adt, double, or float in mixed mode (the update in
 // FP64 from FP32 res and adt, adt_calc in FP32 from x and q rounded, as
-// k_update_mixed and k_adt_calc_mixed).
+// k_update<float> and k_adt_calc_mixed).
 template <class R, bool SOA, bool UPD, bool SAVE>
 __global__ void __launch_bounds__(1024)
     k_direct_chain(const double *qold, double *__restrict q, R *__restrict res,

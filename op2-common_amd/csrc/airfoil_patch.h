@@ -8,12 +8,14 @@
 // q_out, adt_out; the second half the other way round, its update reading the
 // step's first q (qold) from the array it overwrites, each cell its own.  res
 // stays in registers, and the step's copy of q (save_soln) is that array
-// itself.  Per cell and half step 117 bytes (149 in the second) of compulsory
-// traffic, where a direct chain and a res_calc + bres_calc launch move 280-315.
+// itself.  Per cell it moves 128 bytes in a step's first half and 162 in the
+// second at 720,000 cells (counted), where a direct chain and a res_calc +
+// bres_calc launch move 280-315.
 // Measured, one half step against the mean of those launches it replaces:
 // 30.4 against 44.0 us at 720,000 cells (FP64, 256-cell patches), 110 against
-// 173 at 2.88 million (112 MB per 720k cells, 3.7 to 4.2 TB/s), 99 against 144
-// in mixed mode there, and 6.4 against 11.7 at 7,200 cells.
+// 173 at 2.88 million, 99 against 144 in mixed mode there, and 6.4 against 11.7
+// at 7,200 cells; 108 MB a launch at 720,000 cells, 3.65 TB/s, 2,156 MB at 11.5
+// million, 4.6 TB/s.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -131,7 +133,7 @@ __device__ __forceinline__ void stage_cell(const PatchLds<R> &L, int j, const do
 // cells and are done once per staged cell, which leaves 54 operations a side,
 // less than passing the flux through LDS and another barrier), in edge order
 // and from both sides with res_flux's bits, so the results are the sequential
-// executor's.  103 VGPRs, 4 waves per SIMD; capped to 5 or 6 waves it was
+// executor's.  105 VGPRs, 4 waves per SIMD; capped to 5 or 6 waves it was
 // slower (30.4, 30.4, 32.5 us at 720k cells), reading the next patch's lists
 // ahead of the arithmetic changed nothing.  idx0: subtracted from the cell for the reductions' element
 // index (an ensemble member's first cell).  QI: boundary edges with their

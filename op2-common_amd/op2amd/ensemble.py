@@ -67,9 +67,11 @@ def run(sp, niter, warmup=0, batched=True, graphed=True, member_timing=False,
         want_q=False, autotune=False, max_workgroups=0, patch_cells=0, separate_bres=False):
     """Run `niter` time steps of the ensemble `sp` (op2amd_ensemble_run).
 
-    batched: each loop one persistent launch over every member's work items
-    (graphed: the step replayed from a HIP graph), else one launch per loop
-    per member.  autotune: workgroup sizes picked over the first ten steps.
+    batched: each half step (or, where it does not fit, each loop) one
+    persistent launch over every member (graphed: ten steps replayed from a HIP
+    graph), else the same per member.  autotune: workgroup sizes picked over the
+    first ten steps, where the loops have launches of their own; half_steps()
+    counts the half steps launched.
     member_timing: per-member step times (batched: device-clock stamps of
     every work item; looped: HIP events), in member_step_ms (latency inside
     the step) and member_busy_ms (the member's items' spans summed).
