@@ -1652,7 +1652,7 @@ void pack_compact_rows(op_map m, hipStream_t st) {
 
 // The memory of the fused half steps, for the latest owner-plan res_calc and
 // the latest adt_calc's map when they are over the same cells, and the device
-// has room (62 bytes a cell or so).
+// has room (about 66 bytes a cell).
 void make_half_mem() {
   const PendingRes &R = g_last_res;
   const op_map pcell = g_last_pcell.map;
